@@ -204,6 +204,10 @@ void plan_layout(scf_system *S, int want_sx) {
   for (auto &m : S->spec.mol) maxR = std::max(maxR, m.size);
   const int work = W;
   h.threads = work <= 64 ? 64 : (work <= 128 ? 128 : (work <= 256 ? 256 : (work <= 512 ? 512 : 1024)));
+  // the waves of the 1-gradient chains' tiles
+  if (l.gradients == 1 && l.fjc == 1)
+    for (auto &m : S->spec.mol)
+      if (!m.scheduled()) h.threads = std::max(h.threads, std::min(1024, 64 * tile_waves(M, m.size)));
   h.strip_sx = 0;
   h.strip_stride = 0;
   size_t rows = (size_t)2 * maxR * M * D;
@@ -452,7 +456,13 @@ int build(scf_system *S, const Placement *pl) {
   size_t o_G1 = a.take((size_t)nseg * M * D);
   // FP32 segment weights of the grid path's mixed-precision chains (3 gradients)
   size_t o_G1f = l.gradients == 3 ? a.take((size_t)nseg * M * sizeof(float)) : 0;
-  size_t o_Gf = a.take((size_t)maxNR * M * D);
+  // end-point rows; the 1-gradient tiles pad theirs to whole waves, which on
+  // a small lattice is more than the rows themselves
+  size_t gf_doubles = (size_t)maxNR * M;
+  if (l.gradients == 1 && l.fjc == 1)
+    for (auto &m : s.mol)
+      if (!m.scheduled()) gf_doubles = std::max(gf_doubles, tile_store(M, m.chainlength, (int)m.blocks.size(), m.size));
+  size_t o_Gf = a.take(gf_doubles * D);
   size_t o_Gb = a.take((size_t)2 * maxR * M * D);
   size_t o_rho = a.take((size_t)nmm * M * D);
   size_t o_phi = a.take((size_t)nseg * M * D);

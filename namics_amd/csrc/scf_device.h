@@ -27,6 +27,20 @@ constexpr int kMaxMM = 16;
 constexpr int kMaxFjc = 4;   // lattice refinement up to FJC_choices 9
 constexpr int kMaxComp = 2 * kMaxFjc + 1;  // Markov-2 direction components (FJC)
 
+// Wave tiles of the 1-gradient chains (scf_chain1d.h).
+__host__ __device__ constexpr int tile_per_lane(int comps) { return comps == 1 ? 2 : 1; }  // positions per lane
+__host__ __device__ constexpr int tile_halo(int comps) { return comps == 1 ? 8 : 4; }      // per side; steps per exchange
+__host__ __device__ constexpr int tile_own(int comps) { return 64 * tile_per_lane(comps) - 2 * tile_halo(comps); }
+__host__ __device__ constexpr int tile_waves(int M, int comps) { return (M + tile_own(comps) - 1) / tile_own(comps); }
+__host__ __device__ constexpr int tile_rows_every(int comps) { return comps == 1 ? 8 : 4; }
+// End-point storage of one chain in doubles: the first row of every segment
+// of tile_rows_every rows of a block, of every wave's positions, halo
+// included; at most N / rows + blocks segments, of which the chain's first
+// is the segment weight.
+__host__ __device__ constexpr size_t tile_store(int M, int N, int blocks, int comps) {
+  return (size_t)(N / tile_rows_every(comps) + blocks) * tile_waves(M, comps) * 64 * tile_per_lane(comps) * comps;
+}
+
 enum DevStatus : int {
   DS_OK = 0,
   DS_GN = -1,        // GN <= 0 (reference throws -1, src/system.cpp:2398-2402) or not finite

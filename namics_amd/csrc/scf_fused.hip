@@ -95,6 +95,12 @@ __device__ __forceinline__ double wg_max(double v) {
   return t;
 }
 
+}  // namespace nscf
+
+#include "scf_chain1d.h"
+
+namespace nscf {
+
 // ------------------------------------------------------------- propagation
 // Forward recursion of one linear chain, then the backward recursion with
 // the composition law fused into it: rho_block += Gf(s) * Gb(s)
@@ -102,131 +108,6 @@ __device__ __forceinline__ double wg_max(double v) {
 // mol_linear::ComputePhi src/mol_linear.cpp:131-149).  Gf keeps all N rows in
 // HBM; the row being read and the row being written live in LDS when they
 // fit.
-
-// 1-gradient Markov-1 chain, one site per thread (M <= threads): the
-// neighbour indices and lattice weights of the site stay in registers for
-// the whole chain, and the density of a block is accumulated in a register.
-// LG1Planar::propagate (src/LG1Planar.cpp:146-149) and LGrad1::propagate
-// (src/LGrad1.cpp:441-445); a neighbour that falls on a ghost reads the site
-// set_bounds copies there, a missing neighbour (the stencil at the outermost
-// sites) has weight zero.
-__device__ __noinline__ void chain1d_m1(const DevSys &S0, int mo) {
-  CSys &S = uniform_sys(S0);
-  const int M = S.M;
-  const int i = threadIdx.x;
-  const bool active = i < M;
-  const int ii = active ? i : 0;
-  const int i0 = map_x(S, ii);
-  const int im = ii >= 1 ? map_x(S, ii - 1) : i0;
-  const int ip = ii <= M - 2 ? map_x(S, ii + 1) : i0;
-  const bool planar = S.geometry == 0;
-  double wm, w0, wp;
-  if (planar) {
-    wm = S.lambda;
-    w0 = 1.0 - 2.0 * S.lambda;
-    wp = S.lambda;
-  } else {
-    wm = hbm(S.lam_m)[ii];
-    w0 = hbm(S.lam_0)[ii];
-    wp = hbm(S.lam_p)[ii];
-  }
-  if (ii < 1) wm = 0.0;
-  if (ii > M - 2) wp = 0.0;
-  const int b0 = S.mol_block_begin[mo], b1 = S.mol_block_begin[mo + 1];
-  const int N = S.mol_N[mo];
-  gdbl *Gf = hbm(S.Gf);
-  const gdbl *G1 = hbm(S.G1);
-  ldbl *ra = lds_row(0), *rb = lds_row(S.row_stride);
-
-  double g1 = active ? G1[(size_t)S.block_seg[b0] * M + ii] : 0.0;
-  double v = g1;
-  if (active) {
-    Gf[ii] = v;
-    ra[ii] = v;
-  }
-  lds_barrier();
-  ldbl *prev = ra, *next = rb;
-  int s = 1;
-  for (int b = b0; b < b1; b++) {
-    if (b != b0 && active) g1 = G1[(size_t)S.block_seg[b] * M + ii];
-    const int n = S.block_n[b] - (b == b0 ? 1 : 0);
-    for (int j = 0; j < n; j++, s++) {
-      if (active) {
-        double t;
-        if (planar) {
-          t = wm * prev[im];
-          t += w0 * prev[i0];
-        } else {
-          t = w0 * prev[i0];
-          t += wm * prev[im];
-        }
-        t += wp * prev[ip];
-        v = t * g1;
-        Gf[(size_t)s * M + ii] = v;
-        next[ii] = v;
-      }
-      lds_barrier();
-      ldbl *tmp = prev;
-      prev = next;
-      next = tmp;
-    }
-  }
-  // GN = weighted sum of the last end-point distribution (Lattice::ComputeGN)
-  {
-    double acc = 0.0;
-    if (active && ii >= 1 && ii <= S.MX) acc = (planar ? 1.0 : hbm(S.L)[ii]) * v;
-    const double gn = wg_sum(acc);
-    if (threadIdx.x == 0) S0.sc->GN[mo] = gn;
-  }
-  // backward with composition, Gf(s-1) fetched one step ahead.  On a ghost
-  // the composition reads Gf(s) as the reference leaves it: the value
-  // set_bounds copied there when Gf(s) propagated to s+1 (the site i0), and
-  // zero for the last row, whose ghosts ComputeGN's remove_bounds cleared
-  // (src/LGrad1.cpp:213-221,863-874).  Only phitot on the ghosts sees this.
-  ldbl *ga = ra, *gb = rb;
-  const int bl = b1 - 1;
-  const bool ghost = ii < 1 || ii > S.MX;
-  g1 = active ? G1[(size_t)S.block_seg[bl] * M + ii] : 0.0;
-  v = g1;
-  double racc = 0.0, gf = 0.0;
-  if (active) {
-    racc = (ghost ? 0.0 : Gf[(size_t)(N - 1) * M + ii]) * v;
-    ga[ii] = v;
-    if (N >= 2) gf = Gf[(size_t)(N - 2) * M + i0];
-  }
-  lds_barrier();
-  s = N - 2;
-  for (int b = bl; b >= b0; b--) {
-    if (b != bl) {
-      if (active) g1 = G1[(size_t)S.block_seg[b] * M + ii];
-      racc = 0.0;
-    }
-    const int n = S.block_n[b] - (b == bl ? 1 : 0);
-    for (int j = 0; j < n; j++, s--) {
-      if (active) {
-        double t;
-        if (planar) {
-          t = wm * ga[im];
-          t += w0 * ga[i0];
-        } else {
-          t = w0 * ga[i0];
-          t += wm * ga[im];
-        }
-        t += wp * ga[ip];
-        v = t * g1;
-        racc += gf * v;
-        gb[ii] = v;
-        if (s >= 1) gf = Gf[(size_t)(s - 1) * M + i0];
-      }
-      lds_barrier();
-      ldbl *tmp = ga;
-      ga = gb;
-      gb = tmp;
-    }
-    if (active) hbm(S.rho)[(size_t)S.block_mm[b] * M + ii] += racc;
-  }
-  __syncthreads();
-}
 
 // Ring of a first-order chain on a 1-gradient lattice (fjc = 1), one site
 // per thread (mol_linear::ComputePhi src/mol_linear.cpp:35-111).  The first
@@ -236,8 +117,7 @@ __device__ __noinline__ void chain1d_m1(const DevSys &S0, int mo) {
 // in HBM) and ends on x (row N, needed on x only); GN sums the end weights
 // over x.  The merged segment's density on x is G1 times that end weight;
 // the middle blocks' densities come from the backward pass started at
-// delta_x G1, with the same stencil, ghost reads and composition order as
-// chain1d_m1.  Densities and GN collect over the starts in registers.
+// delta_x G1, with the same stencil and ghost reads as a linear chain.  Densities and GN collect over the starts in registers.
 __device__ __noinline__ void chain1d_ring(const DevSys &S0, int mo) {
   CSys &S = uniform_sys(S0);
   const int M = S.M;
@@ -335,165 +215,6 @@ __device__ __noinline__ void chain1d_ring(const DevSys &S0, int mo) {
   if (active) hbm(S.rho)[(size_t)S.block_mm[b0] * M + ii] += racc_a;
   const double gn = wg_sum(gnacc);
   if (threadIdx.x == 0) S0.sc->GN[mo] = gn;
-  __syncthreads();
-}
-
-// Second-order (Markov 2) chain on a 1-gradient simple-cubic lattice, one
-// site per thread (M <= threads), rows in LDS: three direction components per
-// site (+x, lateral, -x), the stencil of m2_step, composition weights
-// (1/6, 4/6, 1/6) (LGrad1::AddPhiS src/LGrad1.cpp:876-910),
-// GN = (G0 + 4 G1 + G2) / 6 (LGrad1::ComputeGN src/LGrad1.cpp:943-955).
-// The arithmetic is chain_markov2's, in the same order; what differs is that
-// no global access sits on a step's critical path: the Boltzmann weight of a
-// block and its density stay in registers (the density is read once at the
-// block's start and written once at its end), and Gf of the backward pass is
-// fetched one step ahead.
-template <int kSPT>
-__device__ __noinline__ void chain1d_m2(const DevSys &S0, int mo) {
-  CSys &S = uniform_sys(S0);
-  const int M = S.M;
-  const int tid = work_tid(S), nt = S.threads;
-  const int R = 3 * M;
-  double P[kMaxComp];
-#pragma unroll
-  for (int k = 0; k < kMaxComp; k++) P[k] = S.mol_P[mo][k];
-  constexpr double wc[3] = {1.0 / 6.0, 4.0 / 6.0, 1.0 / 6.0};
-  int ii[kSPT];
-  bool act[kSPT];
-#pragma unroll
-  for (int k = 0; k < kSPT; k++) {
-    const int w = tid + k * nt;
-    act[k] = w < M;
-    ii[k] = act[k] ? w : 0;
-  }
-  const int b0 = S.mol_block_begin[mo], b1 = S.mol_block_begin[mo + 1];
-  const int N = S.mol_N[mo];
-  gdbl *Gf = hbm(S.Gf);
-  const gdbl *G1 = hbm(S.G1);
-  ldbl *ra = lds_row(0), *rb = lds_row(S.row_stride);
-  double g1[kSPT], o[kSPT][3];
-#pragma unroll
-  for (int k = 0; k < kSPT; k++) {
-    g1[k] = act[k] ? G1[(size_t)S.block_seg[b0] * M + ii[k]] : 0.0;
-    if (act[k])
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        Gf[c * M + ii[k]] = g1[k];
-        ra[c * M + ii[k]] = g1[k];
-      }
-  }
-  lds_barrier();
-  ldbl *prev = ra, *next = rb;
-  int s = 1;
-  for (int b = b0; b < b1; b++) {
-    if (b != b0) {
-#pragma unroll
-      for (int k = 0; k < kSPT; k++)
-        if (act[k]) g1[k] = G1[(size_t)S.block_seg[b] * M + ii[k]];
-    }
-    for (int j = (b == b0 ? 1 : 0); j < S.block_n[b]; j++, s++) {
-#pragma unroll
-      for (int k = 0; k < kSPT; k++) {
-        m2_step<double>(S, (const ldbl *)prev, P, true, ii[k], o[k]);
-#pragma unroll
-        for (int c = 0; c < 3; c++) o[k][c] *= g1[k];
-      }
-      gdbl *gs = Gf + (size_t)s * R;
-#pragma unroll
-      for (int k = 0; k < kSPT; k++)
-        if (act[k])
-#pragma unroll
-          for (int c = 0; c < 3; c++) {
-            gs[c * M + ii[k]] = o[k][c];
-            next[c * M + ii[k]] = o[k][c];
-          }
-      lds_barrier();
-      ldbl *t = prev;
-      prev = next;
-      next = t;
-    }
-  }
-  {
-    double a[3] = {0.0, 0.0, 0.0};
-    const gdbl *gl = Gf + (size_t)(N - 1) * R;
-#pragma unroll
-    for (int k = 0; k < kSPT; k++)
-      if (act[k] && ii[k] >= 1 && ii[k] <= S.MX) {
-        const double wt = site_weight(S0, ii[k]);
-#pragma unroll
-        for (int c = 0; c < 3; c++) a[c] += wt * gl[c * M + ii[k]];
-      }
-    double gn = wg_sum(a[0]);
-    gn += 4.0 * wg_sum(a[1]);
-    gn += wg_sum(a[2]);
-    if (threadIdx.x == 0) S0.sc->GN[mo] = gn / 6.0;
-  }
-  // backward with composition; Gf(s) of every component fetched one step
-  // ahead, the block density in registers
-  ldbl *gbA = ra, *gbB = rb;
-  const int bl = b1 - 1;
-  double racc[kSPT], gf[kSPT][3];
-  {
-    const gdbl *gfl = Gf + (size_t)(N - 1) * R;
-#pragma unroll
-    for (int k = 0; k < kSPT; k++) {
-      g1[k] = act[k] ? G1[(size_t)S.block_seg[bl] * M + ii[k]] : 0.0;
-      racc[k] = act[k] ? hbm(S.rho)[(size_t)S.block_mm[bl] * M + ii[k]] : 0.0;
-      // ghosts: the last row reads zero (ComputeGN's remove_bounds), earlier
-      // rows the components set_bounds(X, Y) paired there (m2_val)
-      const bool ghost = ii[k] < 1 || ii[k] > S.MX;
-      if (act[k]) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          gbA[c * M + ii[k]] = g1[k];
-          racc[k] += wc[c] * (ghost ? 0.0 : gfl[c * M + ii[k]]) * g1[k];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        gf[k][c] = (act[k] && N >= 2) ? m2_val<double>(S, Gf + (size_t)(N - 2) * R, c, ii[k]) : 0.0;
-    }
-  }
-  lds_barrier();
-  s = N - 2;
-  for (int b = bl; b >= b0; b--) {
-    if (b != bl) {
-#pragma unroll
-      for (int k = 0; k < kSPT; k++) {
-        if (act[k]) {
-          hbm(S.rho)[(size_t)S.block_mm[b + 1] * M + ii[k]] = racc[k];
-          g1[k] = G1[(size_t)S.block_seg[b] * M + ii[k]];
-          racc[k] = hbm(S.rho)[(size_t)S.block_mm[b] * M + ii[k]];
-        }
-      }
-    }
-    for (int j = (b == bl ? S.block_n[b] - 2 : S.block_n[b] - 1); j >= 0; j--, s--) {
-#pragma unroll
-      for (int k = 0; k < kSPT; k++) {
-        m2_step<double>(S, (const ldbl *)gbA, P, false, ii[k], o[k]);
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          o[k][c] *= g1[k];
-          racc[k] += wc[c] * gf[k][c] * o[k][c];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < kSPT; k++)
-        if (act[k])
-#pragma unroll
-          for (int c = 0; c < 3; c++) {
-            gbB[c * M + ii[k]] = o[k][c];
-            if (s >= 1) gf[k][c] = m2_val<double>(S, Gf + (size_t)(s - 1) * R, c, ii[k]);
-          }
-      lds_barrier();
-      ldbl *t = gbA;
-      gbA = gbB;
-      gbB = t;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kSPT; k++)
-    if (act[k]) hbm(S.rho)[(size_t)S.block_mm[b0] * M + ii[k]] = racc[k];
   __syncthreads();
 }
 
@@ -1979,6 +1700,51 @@ __device__ __noinline__ double electro_residual(const DevSys &S0, double acc) {
   return acc;
 }
 
+// ------------------------------------------------------------- monomers
+// Molecules of one segment (solvents, ions): their only row is the segment
+// weight, so GN is its weighted sum and the density its square (zero on
+// ghosts, whose last row ComputeGN's remove_bounds clears).  One pass over
+// the sites for all of them, behind one barrier; as one-row chains each cost
+// 6 us of set-up and reductions, of which every system paid at least one.
+__shared__ double s_mono[kMaxMol * 16];  // per-wave partial GN
+
+template <typename Sys>
+__device__ __forceinline__ bool is_monomer(const Sys &S, int mo) {
+  return S.mol_N[mo] == 1 && !S.mol_ring[mo];
+}
+
+__device__ __noinline__ void chain_monomers(const DevSys &S0) {
+  CSys &S = uniform_sys(S0);
+  const int M = S.M, W = n_work_sites(S);
+  const int tid = work_tid(S), nt = S.threads;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  ldbl *part = (ldbl *)s_mono;
+  for (int mo = 0; mo < S.nmol; mo++) {
+    if (!is_monomer(S, mo)) continue;
+    const int b = S.mol_block_begin[mo];
+    const gdbl *g1 = hbm(S.G1) + (size_t)S.block_seg[b] * M;
+    gdbl *rho = hbm(S.rho) + (size_t)S.block_mm[b] * M;
+    double acc = 0.0;
+    for (int w = tid; w < W; w += nt) {
+      int x, y, z;
+      const int i = work_site(S, w, x, y, z);
+      const double g = g1[i];
+      const bool in = is_interior(S, x, y, z);
+      if (in) acc += site_weight(S, i) * g;
+      rho[i] = in ? g * g : 0.0;
+    }
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) part[mo * 16 + wave] = acc;
+  }
+  lds_barrier();
+  if ((int)threadIdx.x < S.nmol && is_monomer(S, (int)threadIdx.x)) {
+    double t = 0.0;
+    for (int w = 0; w < nw; w++) t += part[threadIdx.x * 16 + w];
+    S0.sc->GN[threadIdx.x] = t;
+  }
+  __syncthreads();
+}
+
 // ------------------------------------------------------------- residual
 // One Classical_residual: fields x -> g, densities, norms.  Returns ||g||
 // (or max|g|) to every thread, or a negative value on a status error.
@@ -1999,13 +1765,20 @@ __device__ double fused_residual(const DevSys &S0) {
   }
   __syncthreads();
   const unsigned long long t1 = wall_clock64();
+  bool monomers = false;
+  for (int mo = 0; mo < S.nmol; mo++) monomers = monomers || is_monomer(S, mo);
+  if (monomers) chain_monomers(S0);
   for (int mo = 0; mo < S.nmol; mo++) {
+    if (is_monomer(S, mo)) continue;
     if (S.mol_markov[mo] == 2) {
       const int kind = S.gradients == 3 ? M2_D3 : (S.gradients == 2 ? M2_D2 : (S.lattice_type != 0 ? M2_HEX1 : M2_SC1));
       if (S.use_lds) {
-        if (kind == M2_SC1 && S.M <= S.threads)
-          chain1d_m2<1>(S0, mo);
-        else if (kind == M2_SC1)
+        if (tile_serves(S, mo)) {
+          if (S.geometry == 0)
+            chain1d_tile<3, false>(S0, mo);
+          else
+            chain1d_tile<3, true>(S0, mo);
+        } else if (kind == M2_SC1)
           chain_markov2<true, M2_SC1>(S0, mo);
         else if (kind == M2_HEX1)
           chain_markov2<true, M2_HEX1>(S0, mo);
@@ -2034,8 +1807,11 @@ __device__ double fused_residual(const DevSys &S0) {
       chain_literal(S0, mo);
     } else if (S.strip_sx > 0) {
       chain_strip_dispatch(S0, mo, fp32, fp32 ? sc.lnshift[mo] : 0.0);
-    } else if (S.gradients == 1 && S.fjc == 1 && S.use_lds && S.M <= S.threads) {
-      chain1d_m1(S0, mo);
+    } else if (tile_serves(S, mo)) {
+      if (S.geometry == 0)
+        chain1d_tile<1, false>(S0, mo);
+      else
+        chain1d_tile<1, true>(S0, mo);
     } else if (S.use_lds) {
       chain_markov1<true>(S0, mo);
     } else {

@@ -1203,22 +1203,34 @@ int scf_solve_resident(scf_system *const *systems, int n, scf_solve_info *info) 
     }
   }
   float fused_ms = 0.f;
+  std::vector<SolveRecord> records;  // of the fused systems, in list order, if several
+  size_t at = 0;
   // one launch for all fused systems
   if (!fused.empty()) {
     scf_system *S0 = systems[fused[0]];
     hipStream_t st = S0->stream;
     std::vector<DevSys *> list;
     for (int i : fused) list.push_back(systems[i]->d);
+    const size_t nf = list.size(), list_bytes = (nf * sizeof(DevSys *) + 15) & ~size_t(15);
     DevSys **d_list = S0->d_list;
-    if (list.size() > 1) {
-      HIP_TRY(hipMalloc((void **)&d_list, list.size() * sizeof(DevSys *)));
-      HIP_TRY(hipMemcpy(d_list, list.data(), list.size() * sizeof(DevSys *), hipMemcpyHostToDevice));
+    SolveRecord *d_rec = nullptr;  // several systems: their results come back in one copy
+    hipError_t me = hipSuccess;
+    if (nf > 1) {
+      HIP_TRY(hipMalloc((void **)&d_list, list_bytes + nf * sizeof(SolveRecord)));
+      d_rec = (SolveRecord *)((char *)d_list + list_bytes);
+      me = hipMemcpy(d_list, list.data(), nf * sizeof(DevSys *), hipMemcpyHostToDevice);
     }
-    HIP_TRY(hipEventRecord(S0->ev0, st));
-    hipError_t le = launch_fused(d_list, (int)list.size(), FUSED_SOLVE, threads, lds, st);
+    hipError_t le = me == hipSuccess ? hipEventRecord(S0->ev0, st) : me;
+    if (le == hipSuccess) le = launch_fused(d_list, (int)nf, FUSED_SOLVE, threads, lds, st);
     hipError_t re = hipEventRecord(S0->ev1, st);
+    if (nf > 1) {
+      records.resize(nf);
+      if (le == hipSuccess) le = launch_gather_records(d_list, (int)nf, d_rec, st);
+      if (le == hipSuccess)
+        le = hipMemcpyAsync(records.data(), d_rec, nf * sizeof(SolveRecord), hipMemcpyDeviceToHost, st);
+    }
     hipError_t se = hipStreamSynchronize(st);
-    if (list.size() > 1) hipFree(d_list);
+    if (nf > 1) hipFree(d_list);
     if (le != hipSuccess) return hip_fail(le, "launch_fused");
     if (re != hipSuccess) return hip_fail(re, "hipEventRecord");
     if (se != hipSuccess) return hip_fail(se, "hipStreamSynchronize");
@@ -1242,9 +1254,15 @@ int scf_solve_resident(scf_system *const *systems, int n, scf_solve_info *info) 
       info[i].kernel_ms = ms;
       info[i].solve_ms = ms;
     } else {
-      DevScalars sc;
-      int rc = read_scalars(S, sc);
-      if (rc != SCF_OK) return rc;
+      SolveRecord sc;
+      if (!records.empty()) {
+        sc = records[at++];
+      } else {
+        DevScalars one;
+        int rc = read_scalars(S, one);
+        if (rc != SCF_OK) return rc;
+        sc = {one.iterations, one.status, one.converged, one.fp32_iterations, one.residual, one.t_begin, one.t_end};
+      }
       info[i].iterations = sc.iterations;
       info[i].residual = sc.residual;
       info[i].status = sc.status != DS_OK ? sc.status : (sc.converged ? SCF_OK : SCF_NOT_CONVERGED);
@@ -1257,20 +1275,95 @@ int scf_solve_resident(scf_system *const *systems, int n, scf_solve_info *info) 
   return SCF_OK;
 }
 
+}  // extern "C"
+
+// Host fields of a batch: systems whose fields take at most kPackBytes share
+// one packed copy each way (a copy of its own costs such a system 10-20 us,
+// more than its bytes up to about 64 KiB); larger ones are copied one by one.
+namespace {
+constexpr size_t kPackBytes = 64 * 1024;
+
+struct PackedFields {
+  std::vector<int> which;       // the packed systems
+  std::vector<size_t> offset;   // of each, in doubles
+  std::vector<double> host;
+  DevSys **d_list = nullptr;    // one allocation: list, offsets, fields
+  size_t *d_offset = nullptr;
+  double *d_fields = nullptr;
+
+  ~PackedFields() {
+    if (d_list) (void)hipFree(d_list);
+  }
+  int open(scf_system *const *systems, int n) {
+    size_t total = 0;
+    std::vector<DevSys *> list;
+    for (int i = 0; i < n; i++) {
+      const size_t nvar = (size_t)systems[i]->h.nit * systems[i]->h.M;
+      if (nvar * sizeof(double) > kPackBytes) continue;
+      which.push_back(i);
+      list.push_back(systems[i]->d);
+      offset.push_back(total);
+      total += nvar;
+    }
+    if (which.size() < 2) {
+      which.clear();
+      return SCF_OK;
+    }
+    host.resize(total);
+    const size_t m = which.size();
+    HIP_TRY(hipMalloc((void **)&d_list, m * (sizeof(DevSys *) + sizeof(size_t)) + total * sizeof(double)));
+    d_offset = (size_t *)(d_list + m);
+    d_fields = (double *)(d_offset + m);
+    HIP_TRY(hipMemcpy(d_list, list.data(), m * sizeof(DevSys *), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(d_offset, offset.data(), m * sizeof(size_t), hipMemcpyHostToDevice));
+    return SCF_OK;
+  }
+  size_t count(scf_system *const *systems, size_t k) const {
+    return (size_t)systems[which[k]]->h.nit * systems[which[k]]->h.M;
+  }
+  int upload(scf_system *const *systems, double *const *x) {
+    hipStream_t st = systems[which[0]]->stream;
+    for (size_t k = 0; k < which.size(); k++) {
+      std::memcpy(host.data() + offset[k], x[which[k]], count(systems, k) * sizeof(double));
+      HIP_TRY(hipStreamSynchronize(systems[which[k]]->stream));  // earlier work on its fields
+    }
+    HIP_TRY(hipMemcpyAsync(d_fields, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    HIP_TRY(launch_scatter_fields(d_list, (int)which.size(), d_offset, d_fields, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    return SCF_OK;
+  }
+  int download(scf_system *const *systems, double *const *x) {
+    hipStream_t st = systems[which[0]]->stream;
+    for (size_t k = 0; k < which.size(); k++) HIP_TRY(hipStreamSynchronize(systems[which[k]]->stream));
+    HIP_TRY(launch_gather_fields(d_list, (int)which.size(), d_offset, d_fields, st));
+    HIP_TRY(hipMemcpyAsync(host.data(), d_fields, host.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    for (size_t k = 0; k < which.size(); k++)
+      std::memcpy(x[which[k]], host.data() + offset[k], count(systems, k) * sizeof(double));
+    return SCF_OK;
+  }
+};
+}  // namespace
+
+extern "C" {
+
 int scf_solve_batch(scf_system *const *systems, int n, double *const *x, scf_solve_info *info) {
   if (!systems || n <= 0 || !x || !info) return fail(SCF_E_ARG, "null argument");
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < n; i++)
     if (!systems[i] || !x[i]) return fail(SCF_E_ARG, "null system or field buffer");
-    int rc = scf_upload_fields(systems[i], x[i]);
-    if (rc != SCF_OK) return rc;
-  }
-  int rc = scf_solve_resident(systems, n, info);
+  PackedFields pack;
+  int rc = pack.open(systems, n);
   if (rc != SCF_OK) return rc;
-  for (int i = 0; i < n; i++) {
-    rc = scf_download_fields(systems[i], x[i]);
-    if (rc != SCF_OK) return rc;
-  }
-  return SCF_OK;
+  std::vector<char> packed(n, 0);
+  for (int i : pack.which) packed[i] = 1;
+  for (int i = 0; i < n && rc == SCF_OK; i++)
+    if (!packed[i]) rc = scf_upload_fields(systems[i], x[i]);
+  if (rc == SCF_OK && !pack.which.empty()) rc = pack.upload(systems, x);
+  if (rc == SCF_OK) rc = scf_solve_resident(systems, n, info);
+  for (int i = 0; i < n && rc == SCF_OK; i++)
+    if (!packed[i]) rc = scf_download_fields(systems[i], x[i]);
+  if (rc == SCF_OK && !pack.which.empty()) rc = pack.download(systems, x);
+  return rc;
 }
 
 int scf_get_results(const scf_system *S, scf_results *out) {

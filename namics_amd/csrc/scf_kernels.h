@@ -21,6 +21,17 @@ hipError_t launch_fused_jobs(DevSys *const *slots, int nslots, int chain, const 
 // Static LDS of the fused kernel (bytes), to size the dynamic part.
 size_t fused_static_lds();
 
+// Fields and results of many systems in one packed buffer (scf_batch_io.hip).
+struct SolveRecord {
+  int iterations, status, converged, fp32_iterations;
+  double residual;
+  unsigned long long t_begin, t_end;
+};
+hipError_t launch_scatter_fields(DevSys *const *list, int n, const size_t *offset, const double *packed,
+                                 hipStream_t st);
+hipError_t launch_gather_fields(DevSys *const *list, int n, const size_t *offset, double *packed, hipStream_t st);
+hipError_t launch_gather_records(DevSys *const *list, int n, SolveRecord *rec, hipStream_t st);
+
 // Multi-workgroup path for large lattices (one launch per phase / per
 // propagation step).  Host-driven; see scf_grid.hip.
 struct GridPlan;

@@ -216,11 +216,11 @@ void plan_layout(scf_system *S, int want_sx) {
   // Markov-1 chains, the 9-point stencil, ghosts that map onto interior
   // sites, and the rows of one strip layout in LDS
   const bool strip_ok = l.gradients == 2 && l.fjc == 1 && maxR == 1 && (l.geometry != 0 || l.stencil_full) &&
-                        !S->literal() && !S->has_ring() &&
-                        l.MX + 2 <= 1026 && h.bx1 >= 1 && h.bx1 <= l.MX && h.bxm >= 1 && h.bxm <= l.MX &&
+                        !S->literal() && !S->has_ring() && h.bx1 >= 1 && h.bx1 <= l.MX && h.bxm >= 1 && h.bxm <= l.MX &&
                         h.by1 >= 1 && h.by1 <= l.MY && h.bym >= 1 && h.bym <= l.MY;
+  h.tile2 = strip_ok ? 1 : 0;  // the same lattices, whatever their size
   for (int sx : {8, 4}) {
-    if (!strip_ok || h.strip_sx || l.MX % sx || (want_sx >= 0 && want_sx != sx)) continue;
+    if (!strip_ok || l.MX + 2 > 1026 || h.strip_sx || l.MX % sx || (want_sx >= 0 && want_sx != sx)) continue;
     const int nact = (l.MX / sx) * l.MY;
     if (nact > 1024) continue;
     const int stride = nact <= 256 ? 256 : (nact <= 512 ? 512 : 1024);
@@ -462,6 +462,12 @@ int build(scf_system *S, const Placement *pl) {
   if (l.gradients == 1 && l.fjc == 1)
     for (auto &m : s.mol)
       if (!m.scheduled()) gf_doubles = std::max(gf_doubles, tile_store(M, m.chainlength, (int)m.blocks.size(), m.size));
+  if (l.gradients == 2)
+    for (auto &m : s.mol) {
+      size_t kept = 0;
+      for (auto &b : m.blocks) kept += tile2_segments(b.n);
+      if (!m.scheduled()) gf_doubles = std::max(gf_doubles, kept * M);
+    }
   size_t o_Gf = a.take(gf_doubles * D);
   size_t o_Gb = a.take((size_t)2 * maxR * M * D);
   size_t o_rho = a.take((size_t)nmm * M * D);
@@ -1004,7 +1010,7 @@ int scf_residual(scf_system *S, const double *x, double *g, double *residual) {
   const DevSys &h = S->h;
   const size_t nvar = (size_t)h.nit * h.M;
   HIP_TRY(hipMemcpyAsync(h.x, x, nvar * sizeof(double), hipMemcpyHostToDevice, S->stream));
-  if (S->effective_mode() == SCF_MODE_FUSED) {
+  if (S->mode_among(1) == SCF_MODE_FUSED) {
     HIP_TRY(launch_fused(S->d_list, 1, FUSED_RESIDUAL, h.threads, S->lds_bytes, S->stream));
   } else {
     HIP_TRY(grid_residual(h, S->d, h.partial, S->nb, S->stream));
@@ -1190,13 +1196,17 @@ int scf_solve_resident(scf_system *const *systems, int n, scf_solve_info *info) 
   if (!systems || n <= 0 || !info) return fail(SCF_E_ARG, "null argument");
   std::vector<int> fused;
   size_t lds = 0;
-  int threads = 64;
+  int threads = 64, diis = 0;
   for (int i = 0; i < n; i++) {
     scf_system *S = systems[i];
     if (!S) return fail(SCF_E_ARG, "null system");
     HIP_TRY(hipStreamSynchronize(S->stream));
+    diis += S->newton() ? 0 : 1;
+  }
+  for (int i = 0; i < n; i++) {
+    scf_system *S = systems[i];
     if (S->newton()) continue;
-    if (S->effective_mode() == SCF_MODE_FUSED) {
+    if (S->mode_among(diis) == SCF_MODE_FUSED) {
       fused.push_back(i);
       threads = std::max(threads, S->h.threads);
       lds = std::max(lds, S->lds_bytes);
@@ -1243,7 +1253,7 @@ int scf_solve_resident(scf_system *const *systems, int n, scf_solve_info *info) 
       int rc = method == SOLVER_LBFGS ? lbfgs_solve(S, &info[i])
                                       : (method == SOLVER_BRR ? brr_solve(S, &info[i]) : newton_solve(S, &info[i]));
       if (rc != SCF_OK) return rc;
-    } else if (S->effective_mode() == SCF_MODE_GRID) {
+    } else if (S->mode_among(diis) == SCF_MODE_GRID) {
       HIP_TRY(hipEventRecord(S->ev0, S->stream));
       int rc = grid_solve(S, &info[i]);
       if (rc != SCF_OK) return rc;

@@ -41,6 +41,11 @@ __host__ __device__ constexpr size_t tile_store(int M, int N, int blocks, int co
   return (size_t)(N / tile_rows_every(comps) + blocks) * tile_waves(M, comps) * 64 * tile_per_lane(comps) * comps;
 }
 
+// Segments of the 2-gradient tile chains (scf_tile2d.h): up to kT2H rows of a
+// block, of each of which one row is kept.
+constexpr int kT2H = 8;
+constexpr int tile2_segments(int block_rows) { return (block_rows + kT2H - 1) / kT2H; }
+
 enum DevStatus : int {
   DS_OK = 0,
   DS_GN = -1,        // GN <= 0 (reference throws -1, src/system.cpp:2398-2402) or not finite
@@ -156,6 +161,7 @@ struct DevSys {
   int carry_src[kMaxSeg + 1];  // job queue: field block of the preceding system for each block (-1: zero)
   double mixed_switch;    // residual below which a mixed solve continues in FP64
   double volume;          // weighted interior volume (sum of site weights)
+  int tile2;              // host only: 2-gradient chains can run as tiles over many workgroups (grid path)
   int ckpt;               // 2-gradient strip path: keep every ckpt-th end-point row (0: all rows)
   // ---- scalars and reduction workspace
   DevScalars *sc;

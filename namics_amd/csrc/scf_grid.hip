@@ -504,6 +504,27 @@ __global__ void __launch_bounds__(kGridThreads) k_gn_partial(const DevSys *__res
   if (threadIdx.x == 0) partial[blockIdx.x] = acc;
 }
 
+// A molecule of one segment: GN's partial sums and the density G1 G1 in one
+// pass.
+__global__ void __launch_bounds__(kGridThreads) k_monomer(const DevSys *__restrict__ d, int seg, int mm,
+                                                          double *partial) {
+  CSys &S = uniform_sys(*d);
+  __shared__ double red[kGridThreads / 64];
+  const gdbl *g1 = hbm(S.G1) + (size_t)seg * S.M;
+  gdbl *rho = hbm(S.rho) + (size_t)mm * S.M;
+  double acc = 0;
+  GRID_LOOP(S) {
+    int x, y, z;
+    const int i = work_site(S, w, x, y, z);
+    const double g = g1[i];
+    const bool in = is_interior(S, x, y, z);
+    if (in) acc += site_weight(S, i) * g;
+    rho[i] = in ? g * g : 0.0;
+  }
+  acc = block_sum(acc, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = acc;
+}
+
 // GN of molecule mo from the per-workgroup partials
 __global__ void __launch_bounds__(kGridThreads) k_finalize_gn(const DevSys *__restrict__ d, const double *partial,
                                                                int nparts, int mo) {
@@ -822,6 +843,11 @@ __global__ void __launch_bounds__(kGridThreads) k_diis_combine_dev(const DevSys 
 }
 
 }  // namespace
+}  // namespace nscf
+
+#include "scf_tile2d.h"
+
+namespace nscf {
 
 hipError_t grid_residual(const DevSys &h, DevSys *d, double *partial, int nb, hipStream_t st) {
   hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, st, d);
@@ -865,6 +891,19 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
     if (h.mol_markov[mo] != 1) return hipErrorInvalidValue;
     if (fp32 && !(six && h.G1f)) return hipErrorInvalidValue;
     const int b0 = h.mol_block_begin[mo], b1 = h.mol_block_begin[mo + 1], N = h.mol_N[mo];
+    if (N == 1 && !fp32) {
+      hipLaunchKernelGGL(k_monomer, G, B, 0, st, d, h.block_seg[b0], h.block_mm[b0], partial);
+      hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+      continue;
+    }
+    if (h.tile2) {  // keeps every 8th row at most, with and without checkpoints
+      const Tile2Chain chain(h, mo);
+      const int slot = chain.forward(d, st);
+      hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, slot, partial);
+      hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+      chain.backward(d, st);
+      continue;
+    }
     // block (segment, molecule-segment pair) of every row of the chain
     std::vector<int> rb(N);
     for (int b = b0, r = 0; b < b1; b++)

@@ -11,6 +11,10 @@
 #include "scf_kernels.h"
 #include "scf_spec.h"
 
+// Sites per system and system of a call above which 2-gradient tiles are
+// faster (scf_system::mode_among).
+constexpr int kTileSites = 640;
+
 // One SCF system: its parsed input, device description and HBM arena.
 struct scf_system {
   nscf::SystemSpec spec;
@@ -79,6 +83,24 @@ struct scf_system {
     bool markov2 = false;  // second-order chains run on the fused path only
     for (auto &m : spec.mol) markov2 = markov2 || m.markov == 2;
     return spec.lat.gradients == 3 && !markov2 ? SCF_MODE_GRID : SCF_MODE_FUSED;
+  }
+
+  // The mode of this system when a call solves or evaluates n systems.  A
+  // 2-gradient lattice whose rows do not fit LDS (from about 9800 sites off
+  // the strip path) runs its chains as tiles over many workgroups
+  // (scf_tile2d.h) while the call is small: one after another, such systems
+  // take about 2.5 us per contour index each, while one launch of a workgroup
+  // per system takes 4 ns per site and contour index whatever their number up
+  // to one per CU.  Alone, per evaluation: 101 x 128, N = 100: 5.14 -> 0.38
+  // ms; 128 x 256, N = 400: 49.5 -> 1.09 ms.  Lattices with their rows in LDS
+  // stay with one workgroup each: tiles would be 1.4 to 4 times faster alone,
+  // but a served or batched system gives the bits it gives alone, and there
+  // one workgroup per system has many times the throughput.
+  int mode_among(int n) const {
+    const int m = effective_mode();
+    const bool tiles = m == SCF_MODE_FUSED && mode == SCF_MODE_AUTO && tuned_mode == SCF_MODE_AUTO && h.tile2 &&
+                       h.strip_sx == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;
+    return tiles && (long long)n * kTileSites <= (long long)spec.lat.MX * spec.lat.MY ? SCF_MODE_GRID : m;
   }
 };
 

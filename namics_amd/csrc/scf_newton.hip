@@ -66,7 +66,7 @@ int evaluate(scf_system *S, const double *x, double *g, double *res, int *status
   const size_t nvar = (size_t)h.nit * h.M;
   hipStream_t st = S->stream;
   HIP_TRY(hipMemcpyAsync(h.x, x, nvar * sizeof(double), hipMemcpyHostToDevice, st));
-  if (S->effective_mode() == SCF_MODE_FUSED) {
+  if (S->mode_among(1) == SCF_MODE_FUSED) {
     HIP_TRY(launch_fused(S->d_list, 1, FUSED_RESIDUAL, h.threads, S->lds_bytes, st));
   } else {
     HIP_TRY(grid_residual(h, S->d, h.partial, S->nb, st));

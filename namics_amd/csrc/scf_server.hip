@@ -302,7 +302,7 @@ int scf_server_progress(scf_server *srv, int *queued, int *running) {
       finish(srv, r, sc, host_now(), 0.0);
       continue;
     }
-    if (S->effective_mode() == SCF_MODE_GRID) {
+    if (S->mode_among(1) == SCF_MODE_GRID) {
       std::lock_guard<std::mutex> lk(srv->mu);
       srv->grid_queue.push_back(r);
       srv->cv.notify_one();

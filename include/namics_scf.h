@@ -191,8 +191,9 @@ int scf_system_autotune(scf_system *sys, int evals, scf_tune_report *report);
  * Times `evals` residual evaluations of all n systems in one launch for each
  * end-point storage that applies -- every row (interval 1) and, when every
  * system is on the 2-gradient strip path, every other row with the odd rows
- * recomputed on chip (interval 2, scf_system_set_checkpoint) -- and applies
- * the fastest to all n.  Alone, a system's propagation is bound by its own
+ * recomputed on chip (interval 2, scf_system_set_checkpoint), and, where
+ * those rows together exceed the last-level cache, every third (interval 3)
+ * -- and applies the fastest to all n.  Alone, a system's propagation is bound by its own
  * LDS traffic and recomputing rows costs time; with one system per CU the
  * stored rows saturate HBM and halving them pays.  Results are bit-identical
  * either way.  No counterpart in the reference. */

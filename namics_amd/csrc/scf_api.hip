@@ -233,6 +233,24 @@ void plan_layout(scf_system *S, int want_sx) {
     h.threads = std::max(h.threads, stride);
   }
   h.use_lds = rows <= lds_limit() ? 1 : 0;
+  // the lattice in registers, where its layers have lanes and its columns
+  // waves; the generic chain stays selectable (want_sx = 0) next to a strip
+  // layout
+  h.wave2 = h.wave2_own = 0;
+  bool strip_possible = false;
+  for (int sx : {8, 4}) strip_possible = strip_possible || (strip_ok && l.MX % sx == 0 && (l.MX / sx) * l.MY <= 1024);
+  const int yp = strip_ok && (want_sx != 0 || !strip_possible) ? wave2_layers(l.MY) : 0;
+  if (yp > 0) {
+    const int nw = (l.MX + kWave2Sites / yp - 1) / (kWave2Sites / yp);
+    const size_t edges = (size_t)2 * nw * 128 * yp * D, own = (size_t)1024 * kWave2Sites * D;
+    if (nw <= 16 && edges <= lds_limit()) {
+      h.wave2 = yp;
+      h.wave2_own = edges + own <= lds_limit() ? 1 : 0;
+      h.threads = std::max(h.threads, 64 * nw);
+      h.use_lds = 1;
+      rows = std::max(h.strip_sx || rows <= lds_limit() ? rows : 0, edges + (h.wave2_own ? own : 0));
+    }
+  }
   S->lds_bytes = h.use_lds ? rows : 0;
 }
 
@@ -943,9 +961,19 @@ int scf_autotune_batch(scf_system *const *systems, int n, int evals, scf_batch_t
   }
   // end-point storages every system can hold (the input's save_memory sizes
   // the arena for checkpoints only)
+  // (interval 3 only where the rows of interval 2 outgrow the 256 MB
+  // last-level cache: 256 brushes of 64 x 128 layers, N = 200, 1.29 -> 1.21 ms
+  // per evaluation; within the cache it only adds steps)
   std::vector<int> cand;
-  for (int K : {1, 2}) {
+  double kept = 0;  // bytes of the rows of interval 2
+  for (int i = 0; i < n; i++) {
+    int rows = 0;
+    for (auto &m : systems[i]->spec.mol) rows = std::max(rows, ckpt_rows(m.chainlength, 2) * m.size);
+    kept += (double)rows * systems[i]->spec.lat.M * sizeof(double);
+  }
+  for (int K : {1, 2, 3}) {
     bool fits = K == 1 || strip;
+    if (K == 3 && kept < 256e6) continue;
     for (int i = 0; i < n && fits; i++)
       for (auto &m : systems[i]->spec.mol) fits = fits && ckpt_rows(m.chainlength, K) * m.size <= systems[i]->gf_rows;
     if (fits) cand.push_back(K);

@@ -81,7 +81,7 @@ __device__ __forceinline__ void tile_unfold(const Sys &S, int p, int halo, int &
 // registers (f) just before it composes them, with the next segment's row
 // already on its way: the rows of a 400-layer, N = 2000 second-order chain
 // are 19 MB, which one compute unit cannot stream at the rate of these steps.
-// The recomputation is bit for bit the forward pass.
+// The recomputation repeats the forward pass's steps.
 //
 // A ghost's density (only phitot on the ghosts sees it) composes Gf as
 // set_bounds left it, i.e. the value of the position's site, with Gb as the

@@ -41,6 +41,11 @@ __host__ __device__ constexpr size_t tile_store(int M, int N, int blocks, int co
   return (size_t)(N / tile_rows_every(comps) + blocks) * tile_waves(M, comps) * 64 * tile_per_lane(comps) * comps;
 }
 
+// 2-gradient chains of one workgroup (scf_chain2d.h): sites per thread; the
+// layers per lane for MY layers (0: too many).
+constexpr int kWave2Sites = 8;
+constexpr int wave2_layers(int MY) { return MY <= 64 ? 1 : (MY <= 128 ? 2 : (MY <= 256 ? 4 : 0)); }
+
 // Segments of the 2-gradient tile chains (scf_tile2d.h): up to kT2H rows of a
 // block, of each of which one row is kept.
 constexpr int kT2H = 8;
@@ -161,6 +166,8 @@ struct DevSys {
   int carry_src[kMaxSeg + 1];  // job queue: field block of the preceding system for each block (-1: zero)
   double mixed_switch;    // residual below which a mixed solve continues in FP64
   double volume;          // weighted interior volume (sum of site weights)
+  int wave2;              // 2-gradient chains with the lattice in registers: layers per lane (0: not used)
+  int wave2_own;          // ... with LDS for one recomputed row
   int tile2;              // host only: 2-gradient chains can run as tiles over many workgroups (grid path)
   int ckpt;               // 2-gradient strip path: keep every ckpt-th end-point row (0: all rows)
   // ---- scalars and reduction workspace

@@ -25,7 +25,7 @@ namespace nscf {
 
 // ------------------------------------------------------------- LDS helpers
 __device__ __forceinline__ ldbl *lds_row(int offset) {
-  extern __shared__ double lds_dyn[];
+  extern __shared__ __attribute__((aligned(16))) double lds_dyn[];
   return (ldbl *)(lds_dyn + offset);
 }
 
@@ -98,6 +98,7 @@ __device__ __forceinline__ double wg_max(double v) {
 }  // namespace nscf
 
 #include "scf_chain1d.h"
+#include "scf_chain2d.h"
 
 namespace nscf {
 
@@ -1805,6 +1806,8 @@ __device__ double fused_residual(const DevSys &S0) {
         chain_ring<false>(S0, mo);
     } else if (S.all_sites) {
       chain_literal(S0, mo);
+    } else if (S.wave2 > 0 && !fp32) {
+      chain_wave2_select(S0, mo);
     } else if (S.strip_sx > 0) {
       chain_strip_dispatch(S0, mo, fp32, fp32 ? sc.lnshift[mo] : 0.0);
     } else if (tile_serves(S, mo)) {

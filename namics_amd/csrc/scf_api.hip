@@ -233,6 +233,20 @@ void plan_layout(scf_system *S, int want_sx) {
     h.threads = std::max(h.threads, stride);
   }
   h.use_lds = rows <= lds_limit() ? 1 : 0;
+  // branched molecules on 1-gradient lattices: their rows, the segment weights
+  // and the molecule's densities in LDS
+  h.branch_lds = 0;
+  if (l.gradients == 1 && S->branched()) {
+    size_t need = 0;
+    for (size_t i = 0; i < S->plans.size(); i++)
+      if (S->spec.mol[i].scheduled())
+        need = std::max(need, (size_t)(S->plans[i].rows + h.nseg + (int)S->spec.mol[i].molmon.size()) * M * D);
+    if (need <= lds_limit()) {
+      h.branch_lds = 1;
+      rows = std::max(h.use_lds ? rows : 0, need);
+      h.use_lds = 1;
+    }
+  }
   // the lattice in registers, where its layers have lanes and its columns
   // waves; the generic chain stays selectable (want_sx = 0) next to a strip
   // layout
@@ -499,6 +513,10 @@ int build(scf_system *S, const Placement *pl) {
   size_t o_xR = a.take((size_t)h.m * nvar * D);
   size_t o_xx0 = a.take((size_t)h.m * nvar * D);
   size_t o_x0 = a.take(nvar * D);
+  static_assert(sizeof(BranchStep) == sizeof(BranchOp), "one layout on host and device");
+  size_t n_steps = 0;
+  for (auto &p : S->plans) n_steps += p.forward.size() + p.backward.size();
+  size_t o_br = n_steps ? a.take(n_steps * sizeof(BranchStep)) : 0;
   size_t o_sc = a.take(sizeof(DevScalars));
   // grid path: partial sums (thermo needs 2+nmol columns, DIIS kMaxDIIS)
   const int W = l.gradients == 1 ? M : l.MX * l.MY * (l.gradients == 3 ? l.MZ : 1);
@@ -554,6 +572,23 @@ int build(scf_system *S, const Placement *pl) {
     HIP_TRY(hipMemcpyAsync((void *)h.seg_mask, mask.data(), mask.size() * D, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync((void *)h.ksam, ks.data(), M * D, hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));  // the host vectors end here
+  }
+  if (n_steps) {
+    BranchStep *at = (BranchStep *)(base + o_br);
+    for (int i = 0; i < nmol; i++) {
+      const BranchPlan &p = S->plans[i];
+      h.br_steps[i] = at;
+      h.br_forward[i] = (int)p.forward.size();
+      h.br_backward[i] = (int)p.backward.size();
+      h.br_gn_row[i] = p.gn_row;
+      h.br_rows[i] = p.rows;
+      for (const auto *ops : {&p.forward, &p.backward}) {
+        if (!ops->empty())
+          HIP_TRY(hipMemcpyAsync(at, ops->data(), ops->size() * sizeof(BranchStep), hipMemcpyHostToDevice, st));
+        at += ops->size();
+      }
+    }
+    HIP_TRY(hipStreamSynchronize(st));
   }
   h.x = P(o_x);
   h.g = P(o_g);

@@ -86,6 +86,13 @@ struct JobRecord {
   unsigned long long t_phase[4];  // prepare, chains, densities+residual, rest (device ticks)
 };
 
+// One row operation of a branched molecule's schedule (BranchOp in
+// scf_spec.h, the same layout).
+struct BranchStep {
+  int kind, a, b, c, seg;
+  double f;
+};
+
 struct DevSys {
   // ---- lattice
   int gradients, geometry, lattice_type, stencil_full;
@@ -133,6 +140,11 @@ struct DevSys {
   // host only: the row schedule of a branched molecule (a BranchPlan, see
   // scf_spec.h), null for a linear chain; never read on the device
   const void *branch[kMaxMol];
+  // the same schedule in device memory: forward steps, then backward steps;
+  // the row whose weighted sum is GN, and the rows it uses
+  const BranchStep *br_steps[kMaxMol];
+  int br_forward[kMaxMol], br_backward[kMaxMol], br_gn_row[kMaxMol], br_rows[kMaxMol];
+  int branch_lds;     // the rows of every branched molecule fit LDS (1-gradient lattices)
   double *Gf;         // max over molecules of N * size * M (a branched molecule: its schedule's rows)
   double *Gb;         // 2 * size * M
   double *rho;        // nmm * M (molecule-segment densities)

@@ -20,6 +20,7 @@
 
 #include "scf_device.h"
 #include "scf_kernels.h"
+#include "scf_spec.h"
 
 namespace nscf {
 
@@ -1701,6 +1702,114 @@ __device__ __noinline__ double electro_residual(const DevSys &S0, double acc) {
   return acc;
 }
 
+// ------------------------------------------------------------- branched
+// The row schedule of a branched molecule, dendrimer or comb on a 1-gradient
+// lattice, rows, segment weights and densities in LDS.  A propagation step
+// reads other threads' sites, so it stands between two barriers; everything
+// else works on the thread's own sites.  Bound by the number of operations,
+// each a few LDS accesses (one launch each on the grid path: 1.7 us of kernel
+// and gap).
+__device__ __noinline__ void chain_branched(const DevSys &S0, int mo) {
+  typedef const __attribute__((address_space(4))) BranchStep KStep;
+  CSys &S = uniform_sys(S0);
+  mo = __builtin_amdgcn_readfirstlane(mo);
+  const int M = S.M, tid = work_tid(S), nt = S.threads, nseg = S.nseg;
+  const int mm0 = S.mol_mm_begin[mo], nmm = S.mol_mm_begin[mo + 1] - mm0;
+  ldbl *R = lds_row(0), *W = R + S.br_rows[mo] * M, *D = W + nseg * M;
+  for (int i = tid; i < M; i += nt) {
+    for (int k = 0; k < nseg; k++) W[k * M + i] = hbm(S.G1)[(size_t)k * M + i];
+    for (int c = 0; c < nmm; c++) D[c * M + i] = 0.0;
+  }
+  // one site per thread: its neighbours and lattice weights in registers (as
+  // stencil_prop reads them; a missing neighbour has weight 0)
+  const bool one = S.fjc == 1 && M <= nt, planar = S.geometry == 0;
+  const int x = tid < M ? tid : 0, xl = x >= 1 ? map_x(S, x - 1) : x, xc = map_x(S, x),
+            xr = x <= M - 2 ? map_x(S, x + 1) : x;
+  double wl = S.lambda, wc = 1.0 - 2.0 * S.lambda, wr = S.lambda;
+  if (!planar && one) {
+    wl = hbm(S.lam_m)[x];
+    wc = hbm(S.lam_0)[x];
+    wr = hbm(S.lam_p)[x];
+  }
+  if (x < 1) wl = 0.0;
+  if (x > M - 2) wr = 0.0;
+  auto run = [&](KStep *ops, int n) {
+    // an operation's fields are read while the one before it runs
+    int kind = ops[0].kind, a = ops[0].a, b = ops[0].b, c = ops[0].c, seg = ops[0].seg;
+    double f = ops[0].f;
+    for (int t = 0; t < n; t++) {
+      const int u = t + 1 < n ? t + 1 : t;
+      const int kind1 = ops[u].kind, a1 = ops[u].a, b1 = ops[u].b, c1 = ops[u].c, seg1 = ops[u].seg;
+      const double f1 = ops[u].f;
+      ldbl *ra = R + a * M;
+      const ldbl *rb = R + b * M, *rc = R + c * M, *g1 = W + (seg < 0 ? 0 : seg) * M;
+      if (kind == BR_PROP) {
+        lds_barrier();
+        if (one) {
+          if (tid < M) {
+            double v;
+            if (planar) {
+              v = wl * rb[xl];
+              v += wc * rb[xc];
+            } else {
+              v = wc * rb[xc];
+              v += wl * rb[xl];
+            }
+            v += wr * rb[xr];
+            ra[x] = seg < 0 ? v : v * g1[x];
+          }
+        } else {
+          for (int i = tid; i < M; i += nt) {
+            const double v = stencil_prop<double>(S, rb, i, i, 0, 0);
+            ra[i] = seg < 0 ? v : v * g1[i];
+          }
+        }
+        lds_barrier();
+      } else {
+        ldbl *d = D + c * M;  // (a step counts the molecule's own densities)
+        for (int i = tid; i < M; i += nt) {
+          if (kind == BR_ADDPHI)
+            d[i] += f * ra[i] * rb[i];
+          else if (kind == BR_COPY)
+            ra[i] = rb[i];
+          else if (kind == BR_TIMES)
+            ra[i] = rb[i] * rc[i];
+          else if (kind == BR_INIT)
+            ra[i] = g1[i];
+          else if (kind == BR_ONE)
+            ra[i] = 1.0;
+          else if (kind == BR_TIMES_G1)
+            ra[i] = rb[i] * g1[i];
+          else if (kind == BR_DIV)
+            ra[i] = rb[i] != 0 ? ra[i] / rb[i] : 0.0;
+          else  // BR_DIV_G1
+            ra[i] = g1[i] != 0 ? ra[i] / g1[i] : 0.0;
+        }
+      }
+      kind = kind1;
+      a = a1;
+      b = b1;
+      c = c1;
+      seg = seg1;
+      f = f1;
+    }
+  };
+  KStep *ops = (KStep *)S.br_steps[mo];
+  if (S.br_forward[mo] > 0) run(ops, S.br_forward[mo]);
+  {
+    const ldbl *row = R + S.br_gn_row[mo] * M;
+    double acc = 0.0;
+    for (int i = tid; i < M; i += nt)
+      if (is_interior(S, i, 0, 0)) acc += site_weight(S, i) * row[i];
+    const double gn = wg_sum(acc);
+    if (threadIdx.x == 0) S0.sc->GN[mo] = gn;
+  }
+  if (S.br_backward[mo] > 0) run(ops + S.br_forward[mo], S.br_backward[mo]);
+  for (int i = tid; i < M; i += nt)
+    for (int c = 0; c < nmm; c++) hbm(S.rho)[(size_t)(mm0 + c) * M + i] = D[c * M + i];
+  __syncthreads();
+}
+
 // ------------------------------------------------------------- monomers
 // Molecules of one segment (solvents, ions): their only row is the segment
 // weight, so GN is its weighted sum and the density its square (zero on
@@ -1771,7 +1880,9 @@ __device__ double fused_residual(const DevSys &S0) {
   if (monomers) chain_monomers(S0);
   for (int mo = 0; mo < S.nmol; mo++) {
     if (is_monomer(S, mo)) continue;
-    if (S.mol_markov[mo] == 2) {
+    if (S.br_rows[mo] > 0) {
+      chain_branched(S0, mo);
+    } else if (S.mol_markov[mo] == 2) {
       const int kind = S.gradients == 3 ? M2_D3 : (S.gradients == 2 ? M2_D2 : (S.lattice_type != 0 ? M2_HEX1 : M2_SC1));
       if (S.use_lds) {
         if (tile_serves(S, mo)) {

@@ -884,8 +884,10 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
         hipLaunchKernelGGL(k_branch_op, G, B, 0, st, d, o.kind, o.a, o.b, o.c, o.seg, o.f);
       hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, plan.gn_row, partial);
       hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+      // (an operation counts the molecule's own densities)
       for (const BranchOp &o : plan.backward)
-        hipLaunchKernelGGL(k_branch_op, G, B, 0, st, d, o.kind, o.a, o.b, o.c, o.seg, o.f);
+        hipLaunchKernelGGL(k_branch_op, G, B, 0, st, d, o.kind, o.a, o.b,
+                           o.kind == BR_ADDPHI ? h.mol_mm_begin[mo] + o.c : o.c, o.seg, o.f);
       continue;
     }
     if (h.mol_markov[mo] != 1) return hipErrorInvalidValue;

@@ -487,7 +487,6 @@ int build(scf_system *S, const Placement *pl) {
   size_t o_g = a.take(nvar * D);
   size_t o_G1 = a.take((size_t)nseg * M * D);
   // FP32 segment weights of the grid path's mixed-precision chains (3 gradients)
-  size_t o_G1f = l.gradients == 3 ? a.take((size_t)nseg * M * sizeof(float)) : 0;
   // end-point rows; the 1-gradient tiles pad theirs to whole waves, which on
   // a small lattice is more than the rows themselves
   size_t gf_doubles = (size_t)maxNR * M;
@@ -593,7 +592,6 @@ int build(scf_system *S, const Placement *pl) {
   h.x = P(o_x);
   h.g = P(o_g);
   h.G1 = P(o_G1);
-  h.G1f = l.gradients == 3 ? (float *)P(o_G1f) : nullptr;
   h.Gf = P(o_Gf);
   h.Gb = P(o_Gb);
   h.rho = P(o_rho);

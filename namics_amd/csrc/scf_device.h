@@ -136,7 +136,6 @@ struct DevSys {
   // ---- work arrays (device)
   double *x, *g;
   double *G1;         // nseg * M
-  float *G1f;         // nseg * M (3-gradient grid path): FP32 segment weights times the gauge factor e^c
   // host only: the row schedule of a branched molecule (a BranchPlan, see
   // scf_spec.h), null for a linear chain; never read on the device
   const void *branch[kMaxMol];

@@ -7,6 +7,7 @@
 // partial sums in HBM, summed in workgroup order by one thread.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "scf_device.h"
@@ -241,21 +242,6 @@ __global__ void __launch_bounds__(kGridThreads) k_step_bwd(const DevSys *__restr
   }
 }
 
-// 3-gradient steps (LGrad3::propagate src/LGrad3.cpp:731-743): one thread
-// per site of an x-plane, (y, z) flattened with z fastest, so every load is
-// coalesced; a workgroup covers part of one plane.
-__device__ __forceinline__ double stencil3(CSys &S, const gdbl *__restrict__ g, int x, int y, int z) {
-  const int JX = S.JX, JY = S.JY;
-  const int bx = x * JX, by = y * JY;
-  double v = g[map_x(S, x - 1) * JX + by + z];
-  v += g[map_x(S, x + 1) * JX + by + z];
-  v += g[bx + map_y(S, y - 1) * JY + z];
-  v += g[bx + map_y(S, y + 1) * JY + z];
-  v += g[bx + by + map_z(S, z - 1)];
-  v += g[bx + by + map_z(S, z + 1)];
-  return v * (1.0 / 6.0);
-}
-
 // Workgroups are handed to the 8 XCDs round-robin by dispatch order.  The
 // 3-gradient steps renumber them so that each XCD takes a contiguous run of
 // x-planes: the x-1 / x+1 planes a workgroup reads are then mostly read by
@@ -267,193 +253,16 @@ __device__ __forceinline__ int xcd_block_id() {
   return (c < r ? c * (q + 1) : r * (q + 1) + (c - r) * q) + k;
 }
 
-__device__ __forceinline__ void xcd_plane_block(int &xplane, int &bx) {
-  const int L = xcd_block_id();
-  xplane = L / gridDim.x;
-  bx = L - xplane * gridDim.x;
-}
-
-__global__ void __launch_bounds__(kGridThreads) k_step3_fwd(const DevSys *__restrict__ d, int src, int dst,
-                                                            int seg) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const gdbl *prev = hbm(S.Gf) + (size_t)src * M;
-  hbm(S.Gf)[(size_t)dst * M + i] = stencil3(S, prev, x, y, z) * hbm(S.G1)[(size_t)seg * M + i];
-}
-
-__global__ void __launch_bounds__(kGridThreads) k_step3_bwd(const DevSys *__restrict__ d, int slot, int seg, int mm,
-                                                            int src) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const gdbl *gb = hbm(S.Gb) + (size_t)src * M;
-  const double v = stencil3(S, gb, x, y, z) * hbm(S.G1)[(size_t)seg * M + i];
-  hbm(S.Gb)[(size_t)(1 - src) * M + i] = v;
-  gdbl *rho = hbm(S.rho) + (size_t)mm * M;
-  rho[i] += hbm(S.Gf)[(size_t)slot * M + i] * v;
-}
-
-// The forward pass's first and last 6-point steps with the neighbouring
-// one-row phases folded in: the first step reads row 0 from the segment
-// weights and stores it (k_row_init), the last one also starts the
-// backward pass (k_bwd_first: Gb = G1, rho += G(N-1) G1).  Same arithmetic
-// as the separate launches, one launch less each.
-template <bool kFirst, bool kLast>
-__global__ void __launch_bounds__(kGridThreads) k_step3_fwd_x(const DevSys *__restrict__ d, int src, int dst,
-                                                              int seg, int seg0, int slot0, int mm) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const gdbl *prev = kFirst ? hbm(S.G1) + (size_t)seg0 * M : hbm(S.Gf) + (size_t)src * M;
-  const double g = hbm(S.G1)[(size_t)seg * M + i];
-  const double v = stencil3(S, prev, x, y, z) * g;
-  hbm(S.Gf)[(size_t)dst * M + i] = v;
-  if (kFirst) hbm(S.Gf)[(size_t)slot0 * M + i] = prev[i];
-  if (kLast) {
-    hbm(S.Gb)[i] = g;
-    hbm(S.rho)[(size_t)mm * M + i] += v * g;
-  }
-}
-
 // ---- FP32 end points on the 6-point 3-gradient steps (mixed precision).
 // Rows hold G(s) e^{c (s+1)} in FP32 (forward) and G(s) e^{c (N-s)}
 // (backward), where c = -ln(GN / V) / N is the molecule's gauge shift from
-// the latest GN: the segment weights are G1' = G1 e^c (k_g1_shift32), so
-// the shifted end points average about one per site whatever N and the
-// fields.  GN and the composition are taken back to FP64 and unshifted
-// (GN = GN' e^{-cN}; rho += Gf' Gb' e^{-c(N+1)}).  The steps move 12 B per
-// site (forward) and 28 B (backward, rho in FP64) instead of 24 and 48.
+// the latest GN: the segment weights are G1' = G1 e^c, so the shifted end
+// points average about one per site whatever N and the fields.  GN and the
+// composition are taken back to FP64 and unshifted (GN = GN' e^{-cN};
+// rho += Gf' Gb' e^{-c(N+1)}).  A molecule of one segment stays in FP64.
 typedef __attribute__((address_space(1))) float gflt;
 __device__ __forceinline__ gflt *hbmf(float *p) { return (gflt *)p; }
 __device__ __forceinline__ const gflt *hbmf(const float *p) { return (const gflt *)p; }
-
-__device__ __forceinline__ float stencil3f(CSys &S, const gflt *__restrict__ g, int x, int y, int z) {
-  const int JX = S.JX, JY = S.JY;
-  const int bx = x * JX, by = y * JY;
-  float v = g[map_x(S, x - 1) * JX + by + z];
-  v += g[map_x(S, x + 1) * JX + by + z];
-  v += g[bx + map_y(S, y - 1) * JY + z];
-  v += g[bx + map_y(S, y + 1) * JY + z];
-  v += g[bx + by + map_z(S, z - 1)];
-  v += g[bx + by + map_z(S, z + 1)];
-  return v * (1.0f / 6.0f);
-}
-
-// G1' = G1 e^c of every segment, for molecule mo's chain
-__global__ void __launch_bounds__(kGridThreads) k_g1_shift32(const DevSys *__restrict__ d, int mo) {
-  CSys &S = uniform_sys(*d);
-  const double es = exp(S.sc->lnshift[mo]);
-  const int n = S.nseg * S.M;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    hbmf(S.G1f)[i] = (float)(hbm(S.G1)[i] * es);
-}
-
-__global__ void __launch_bounds__(kGridThreads) k_row_init32(const DevSys *__restrict__ d, int seg) {
-  CSys &S = uniform_sys(*d);
-  const gflt *g1 = hbmf(S.G1f) + (size_t)seg * S.M;
-  gflt *gf = hbmf((float *)S.Gf);
-  GRID_LOOP(S) {
-    int x, y, z;
-    const int i = work_site(S, w, x, y, z);
-    gf[i] = g1[i];
-  }
-}
-
-__global__ void __launch_bounds__(kGridThreads) k_step3_fwd32(const DevSys *__restrict__ d, int src, int dst,
-                                                              int seg) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const gflt *prev = hbmf((const float *)S.Gf) + (size_t)src * M;
-  hbmf((float *)S.Gf)[(size_t)dst * M + i] = stencil3f(S, prev, x, y, z) * hbmf(S.G1f)[(size_t)seg * M + i];
-}
-
-// k_step3_fwd_x with FP32 end points
-template <bool kFirst, bool kLast>
-__global__ void __launch_bounds__(kGridThreads) k_step3_fwd32_x(const DevSys *__restrict__ d, int src, int dst,
-                                                                int seg, int seg0, int slot0, int mm, int mo) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const gflt *prev = kFirst ? hbmf(S.G1f) + (size_t)seg0 * M : hbmf((const float *)S.Gf) + (size_t)src * M;
-  const float g = hbmf(S.G1f)[(size_t)seg * M + i];
-  const float v = stencil3f(S, prev, x, y, z) * g;
-  hbmf((float *)S.Gf)[(size_t)dst * M + i] = v;
-  if (kFirst) hbmf((float *)S.Gf)[(size_t)slot0 * M + i] = prev[i];
-  if (kLast) {
-    const double unshift = exp(-S.sc->lnshift[mo] * (S.mol_N[mo] + 1));
-    hbmf((float *)S.Gb)[i] = g;
-    hbm(S.rho)[(size_t)mm * M + i] += (double)v * (double)g * unshift;
-  }
-}
-
-// first backward row (G1') and its composition, unshifted
-__global__ void __launch_bounds__(kGridThreads) k_bwd_first32(const DevSys *__restrict__ d, int slot, int seg,
-                                                              int mm, int mo) {
-  CSys &S = uniform_sys(*d);
-  const int M = S.M;
-  const double unshift = exp(-S.sc->lnshift[mo] * (S.mol_N[mo] + 1));
-  const gflt *g1 = hbmf(S.G1f) + (size_t)seg * M;
-  const gflt *gf = hbmf((const float *)S.Gf) + (size_t)slot * M;
-  gdbl *rho = hbm(S.rho) + (size_t)mm * M;
-  GRID_LOOP(S) {
-    int x, y, z;
-    const int i = work_site(S, w, x, y, z);
-    const float v = g1[i];
-    hbmf((float *)S.Gb)[i] = v;
-    rho[i] += (double)gf[i] * (double)v * unshift;
-  }
-}
-
-__global__ void __launch_bounds__(kGridThreads) k_step3_bwd32(const DevSys *__restrict__ d, int slot, int seg,
-                                                              int mm, int src, int mo) {
-  CSys &S = uniform_sys(*d);
-  const int MZ = S.MZ, M = S.M;
-  int xp, bx;
-  xcd_plane_block(xp, bx);
-  const int p = bx * kGridThreads + threadIdx.x;
-  if (p >= S.MY * MZ) return;
-  const int yy = p / MZ;
-  const int x = xp + 1, y = yy + 1, z = p - yy * MZ + 1;
-  const int i = x * S.JX + y * S.JY + z;
-  const double unshift = exp(-S.sc->lnshift[mo] * (S.mol_N[mo] + 1));
-  const gflt *gb = hbmf((const float *)S.Gb) + (size_t)src * M;
-  const float v = stencil3f(S, gb, x, y, z) * hbmf(S.G1f)[(size_t)seg * M + i];
-  hbmf((float *)S.Gb)[(size_t)(1 - src) * M + i] = v;
-  gdbl *rho = hbm(S.rho) + (size_t)mm * M;
-  rho[i] += (double)hbmf((const float *)S.Gf)[(size_t)slot * M + i] * (double)v * unshift;
-}
 
 __global__ void __launch_bounds__(kGridThreads) k_gn_partial32(const DevSys *__restrict__ d, int slot,
                                                                double *partial) {
@@ -849,11 +658,6 @@ __global__ void __launch_bounds__(kGridThreads) k_diis_combine_dev(const DevSys 
 
 namespace nscf {
 
-hipError_t grid_residual(const DevSys &h, DevSys *d, double *partial, int nb, hipStream_t st) {
-  hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, st, d);
-  return grid_residual_body(h, d, partial, nb, st);
-}
-
 // End-point storage of the grid path.  With every row kept (ckpt <= 1) row
 // s of the forward recursion is Gf slot s.  With checkpoints every K rows
 // (the reference's save_memory, src/molecule.cpp:2300-2446) the slots hold
@@ -869,11 +673,21 @@ struct RowSlots {
   int operator()(int r) const { return K <= 1 ? r : (r % K == 0 ? r / K : nck + r % K - 1); }
 };
 
+}  // namespace nscf
+
+#include "scf_box3d.h"
+
+namespace nscf {
+
+hipError_t grid_residual(const DevSys &h, DevSys *d, double *partial, int nb, hipStream_t st) {
+  hipLaunchKernelGGL(k_reset_status, dim3(1), dim3(1), 0, st, d);
+  return grid_residual_body(h, d, partial, nb, st);
+}
+
 hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int nb, hipStream_t st, bool fp32) {
   const dim3 B(kGridThreads), G(nb);
-  const dim3 G3((h.MY * h.MZ + kGridThreads - 1) / kGridThreads, h.MX);
-  // the plane-mapped 6-point kernels serve the default simple-cubic 3-D
-  // stencil; the 26-neighbour stencils go through the generic step
+  // the box tiles serve the default simple-cubic 3-D stencil; the
+  // 26-neighbour stencils go through the generic step
   const bool six = h.gradients == 3 && h.stencil_full && h.lattice_type == 0;
   hipLaunchKernelGGL(k_prepare, G, B, 0, st, d);
   for (int mo = 0; mo < h.nmol; mo++) {
@@ -891,9 +705,9 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
       continue;
     }
     if (h.mol_markov[mo] != 1) return hipErrorInvalidValue;
-    if (fp32 && !(six && h.G1f)) return hipErrorInvalidValue;
+    if (fp32 && !six) return hipErrorInvalidValue;
     const int b0 = h.mol_block_begin[mo], b1 = h.mol_block_begin[mo + 1], N = h.mol_N[mo];
-    if (N == 1 && !fp32) {
+    if (N == 1) {
       hipLaunchKernelGGL(k_monomer, G, B, 0, st, d, h.block_seg[b0], h.block_mm[b0], partial);
       hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
       continue;
@@ -906,75 +720,32 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
       chain.backward(d, st);
       continue;
     }
-    // block (segment, molecule-segment pair) of every row of the chain
-    std::vector<int> rb(N);
-    for (int b = b0, r = 0; b < b1; b++)
-      for (int j = 0; j < h.block_n[b]; j++) rb[r++] = b;
     const RowSlots loc{h.ckpt, h.ckpt > 1 ? (N + h.ckpt - 1) / h.ckpt : N};
+    if (six) {
+      const BoxChain chain(h, mo, fp32);
+      const hipError_t e = chain.run(st, [&] {
+        if (fp32) {
+          hipLaunchKernelGGL(k_gn_partial32, G, B, 0, st, d, loc(N - 1), partial);
+          hipLaunchKernelGGL(k_finalize_gn32, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+        } else {
+          hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, loc(N - 1), partial);
+          hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+        }
+      });
+      if (e != hipSuccess) return e;
+      continue;
+    }
+    // block (segment, molecule-segment pair) of every row of the chain
+    std::vector<int> rb;
+    for (int b = b0; b < b1; b++) rb.insert(rb.end(), h.block_n[b], b);
     auto fwd = [&](int r) {
-      const int seg = h.block_seg[rb[r]];
-      if (fp32)
-        hipLaunchKernelGGL(k_step3_fwd32, G3, B, 0, st, d, loc(r - 1), loc(r), seg);
-      else if (six)
-        hipLaunchKernelGGL(k_step3_fwd, G3, B, 0, st, d, loc(r - 1), loc(r), seg);
-      else
-        hipLaunchKernelGGL(k_step_fwd, G, B, 0, st, d, loc(r - 1), loc(r), seg);
+      hipLaunchKernelGGL(k_step_fwd, G, B, 0, st, d, loc(r - 1), loc(r), h.block_seg[rb[r]]);
     };
-    // 6-point chains fold the row init into the first step and the first
-    // backward row into the last one
-    const bool fold = six && N >= 2;
-    const int seg0 = h.block_seg[b0], segN = h.block_seg[rb[N - 1]], mmN = h.block_mm[rb[N - 1]];
-    auto fwd_folded = [&](int r) {
-      const bool first = r == 1, last = r == N - 1;
-      const int seg = h.block_seg[rb[r]];
-      if (fp32) {
-        if (first && last)
-          hipLaunchKernelGGL((k_step3_fwd32_x<true, true>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0, loc(0),
-                             mmN, mo);
-        else if (first)
-          hipLaunchKernelGGL((k_step3_fwd32_x<true, false>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0, loc(0),
-                             mmN, mo);
-        else if (last)
-          hipLaunchKernelGGL((k_step3_fwd32_x<false, true>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0,
-                             loc(0), mmN, mo);
-        else
-          fwd(r);
-      } else {
-        if (first && last)
-          hipLaunchKernelGGL((k_step3_fwd_x<true, true>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0, loc(0),
-                             mmN);
-        else if (first)
-          hipLaunchKernelGGL((k_step3_fwd_x<true, false>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0, loc(0),
-                             mmN);
-        else if (last)
-          hipLaunchKernelGGL((k_step3_fwd_x<false, true>), G3, B, 0, st, d, loc(r - 1), loc(r), seg, seg0, loc(0),
-                             mmN);
-        else
-          fwd(r);
-      }
-    };
-    if (fp32) hipLaunchKernelGGL(k_g1_shift32, G, B, 0, st, d, mo);
-    if (!fold) {
-      if (fp32)
-        hipLaunchKernelGGL(k_row_init32, G, B, 0, st, d, seg0);
-      else
-        hipLaunchKernelGGL(k_row_init, G, B, 0, st, d, seg0);
-    }
-    for (int r = 1; r < N; r++) {
-      if (fold)
-        fwd_folded(r);
-      else
-        fwd(r);
-    }
-    if (fp32) {
-      hipLaunchKernelGGL(k_gn_partial32, G, B, 0, st, d, loc(N - 1), partial);
-      hipLaunchKernelGGL(k_finalize_gn32, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
-      if (!fold) hipLaunchKernelGGL(k_bwd_first32, G, B, 0, st, d, loc(N - 1), segN, mmN, mo);
-    } else {
-      hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, loc(N - 1), partial);
-      hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
-      if (!fold) hipLaunchKernelGGL(k_bwd_first, G, B, 0, st, d, loc(N - 1), segN, mmN);
-    }
+    hipLaunchKernelGGL(k_row_init, G, B, 0, st, d, h.block_seg[b0]);
+    for (int r = 1; r < N; r++) fwd(r);
+    hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, loc(N - 1), partial);
+    hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
+    hipLaunchKernelGGL(k_bwd_first, G, B, 0, st, d, loc(N - 1), h.block_seg[rb[N - 1]], h.block_mm[rb[N - 1]]);
     int src = 0, seg_in_buffer = h.ckpt > 1 ? (N - 1) / h.ckpt : -1;
     for (int s = N - 2; s >= 0; s--) {
       if (h.ckpt > 1 && s / h.ckpt != seg_in_buffer) {
@@ -984,12 +755,7 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
         for (int r = a0 + 1; r < a0 + h.ckpt && r < N; r++) fwd(r);
       }
       const int b = rb[s];
-      if (fp32)
-        hipLaunchKernelGGL(k_step3_bwd32, G3, B, 0, st, d, loc(s), h.block_seg[b], h.block_mm[b], src, mo);
-      else if (six)
-        hipLaunchKernelGGL(k_step3_bwd, G3, B, 0, st, d, loc(s), h.block_seg[b], h.block_mm[b], src);
-      else
-        hipLaunchKernelGGL(k_step_bwd, G, B, 0, st, d, loc(s), h.block_seg[b], h.block_mm[b], src);
+      hipLaunchKernelGGL(k_step_bwd, G, B, 0, st, d, loc(s), h.block_seg[b], h.block_mm[b], src);
       src = 1 - src;
     }
   }

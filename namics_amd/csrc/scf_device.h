@@ -1456,6 +1456,48 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
+// v and the value 32 (16) lanes away, added or the larger.
+__device__ __forceinline__ double half_swap(double v, bool max, int by) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  unsigned l0, l1, h0, h1;
+  if (by == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  }
+  const double p = __longlong_as_double((long long)(((unsigned long long)h0 << 32) | l0));
+  const double q = __longlong_as_double((long long)(((unsigned long long)h1 << 32) | l1));
+  return max ? fmax(p, q) : p + q;
+}
+
+// Sum (largest) of the 64 lanes of a wave, on every lane: the lanes 32, 16,
+// 8, 4, 2, 1 apart in turn, in registers (the swap of halves and DPP), where
+// the same tree over LDS exchanges is a chain of six round trips: 183 for 471
+// clocks, the same bits.
+__device__ __forceinline__ double wave_sum(double v) {
+  v = half_swap(v, false, 32);
+  v = half_swap(v, false, 16);
+  v += dpp_f64<0x128>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x4E>(v);
+  v += dpp_f64<0xB1>(v);
+  return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = half_swap(v, true, 32);
+  v = half_swap(v, true, 16);
+  v = fmax(v, dpp_f64<0x128>(v));
+  v = fmax(v, dpp_f64<0x124>(v));
+  v = fmax(v, dpp_f64<0x4E>(v));
+  v = fmax(v, dpp_f64<0xB1>(v));
+  return v;
+}
+
 // DIIS coefficients on the device by one wavefront: c = A^-1 (1..1) / sum,
 // A is the kd x kd Gram matrix (leading dimension kd, kd <= kMaxDIIS = 16).
 // Lane r holds row r; Gauss-Jordan elimination with partial pivoting (pivot
@@ -1520,12 +1562,10 @@ __device__ __forceinline__ bool wave_diis_coefficients(const double *A, int n, d
       if (c == pc) d = row[c];
     x = rhs / d;
   }
-  double sum = lane < n ? x : 0.0;
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  int anybad = (bad || (lane < n && (pc < 0 || x != x))) ? 1 : 0;
-  for (int off = 32; off > 0; off >>= 1) anybad |= __shfl_xor(anybad, off, 64);
+  const double sum = wave_sum(lane < n ? x : 0.0);
+  const bool anybad = __any(bad || (lane < n && (pc < 0 || x != x)));
   if (lane < n && pc >= 0) C[pc] = x / sum;
-  return anybad == 0 && sum == sum && sum != 0.0;
+  return !anybad && sum == sum && sum != 0.0;
 }
 
 // Record the new Gram row (SFNewton::DIIS src/sfnewton.cpp:837-867): shift

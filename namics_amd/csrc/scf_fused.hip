@@ -71,7 +71,7 @@ __device__ __forceinline__ int work_tid(const Sys &S) {
 // ------------------------------------------------------------- reductions
 // Workgroup sum; every thread gets the same value (summed in a fixed order).
 __device__ __forceinline__ double wg_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = wave_sum(v);
   ldbl *red = (ldbl *)s_red;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   lds_barrier();
@@ -79,12 +79,13 @@ __device__ __forceinline__ double wg_sum(double v) {
   lds_barrier();
   double t = 0;
   const int nw = blockDim.x >> 6;
-  for (int w = 0; w < nw; w++) t += red[w];
+#pragma unroll  // (every read in flight at once; adding an absent wave's zero moves no bit)
+  for (int w = 0; w < 16; w++) t += w < nw ? red[w] : 0.0;
   return t;
 }
 
 __device__ __forceinline__ double wg_max(double v) {
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+  v = wave_max(v);
   ldbl *red = (ldbl *)s_red;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   lds_barrier();
@@ -92,7 +93,8 @@ __device__ __forceinline__ double wg_max(double v) {
   lds_barrier();
   double t = 0;
   const int nw = blockDim.x >> 6;
-  for (int w = 0; w < nw; w++) t = fmax(t, red[w]);
+#pragma unroll
+  for (int w = 0; w < 16; w++) t = fmax(t, w < nw ? red[w] : 0.0);
   return t;
 }
 
@@ -1843,7 +1845,7 @@ __device__ __noinline__ void chain_monomers(const DevSys &S0) {
       if (in) acc += site_weight(S, i) * g;
       rho[i] = in ? g * g : 0.0;
     }
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    acc = wave_sum(acc);
     if (lane == 0) part[mo * 16 + wave] = acc;
   }
   lds_barrier();
@@ -2113,8 +2115,7 @@ __device__ __noinline__ void diis_update_dots(const DevSys &S0, int k, int kd, d
 #pragma unroll
   for (int i = 0; i < kMaxDIIS; i++) {
     if (i < kd) {
-      double t = i < kd - 1 ? acc[i < kMaxDIIS - 1 ? i : 0] : self;
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      const double t = wave_sum(i < kd - 1 ? acc[i < kMaxDIIS - 1 ? i : 0] : self);
       if (lane == 0) dred[i * 16 + wave] = t;
     }
   }

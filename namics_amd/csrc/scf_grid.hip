@@ -20,7 +20,7 @@ namespace {
 constexpr int kGridThreads = 256;
 
 __device__ __forceinline__ double block_sum(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wave] = v;
@@ -39,8 +39,7 @@ __device__ __forceinline__ void block_sums_store(const double *acc, int ncols, d
 #pragma unroll
   for (int i = 0; i < kMaxDIIS; i++) {
     if (i < ncols) {
-      double v = acc[i];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      const double v = wave_sum(acc[i]);
       if (lane == 0) red[i * nw + wave] = v;
     }
   }
@@ -53,7 +52,7 @@ __device__ __forceinline__ void block_sums_store(const double *acc, int ncols, d
 }
 
 __device__ __forceinline__ double block_max(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+  v = wave_max(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wave] = v;

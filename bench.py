@@ -55,6 +55,13 @@ def stored_rows(N, ckpt):
     return N if ckpt <= 1 else -(-N // ckpt)
 
 
+def end_point_bytes(desc, mol, ckpt, w, W):
+    """Bytes of a molecule's stored rows, written once and read once."""
+    size = mol.get("size", 1)
+    every = (8 if size == 1 else 4) if desc["gradients"] == 1 else ckpt
+    return 2 * w * size * W * stored_rows(mol["chainlength"], every)
+
+
 def hbm_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     """Bytes one residual evaluation plus one DIIS update must move through
     HBM on the fused path, each array read or written once (what a perfect
@@ -64,7 +71,9 @@ def hbm_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     * end-point rows: every stored row written once in the forward pass and
       read once in the backward pass, 2 w per stored site and row
       (w = 4 B with FP32 propagators), over the sites the chain kernel stores
-      (interior sites on 2-gradient lattices, all sites on 1 gradient);
+      (interior sites on 2-gradient lattices, all sites on 1 gradient, where
+      every 8th row of a first-order and every 4th of a second-order chain is
+      stored and the rows between are recomputed on chip);
     * per-site arrays of the evaluation (8 B per site each): fields x read by
       the Boltzmann-weight pass and the residual (2 nit rows), G1 written
       (nseg) and read by every block of the forward and backward passes
@@ -82,7 +91,7 @@ def hbm_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     g = desc["gradients"]
     M = desc["M"]
     W = M if g == 1 else desc["MX"] * (desc["MY"] if g >= 2 else 1) * (desc["MZ"] if g == 3 else 1)
-    gf = sum(2 * w * m.get("size", 1) * W * stored_rows(m["chainlength"], ckpt) for m in desc["molecules"])
+    gf = sum(end_point_bytes(desc, m, ckpt, w, W) for m in desc["molecules"])
     nit = len(desc["fields"])
     nseg = len(desc["segments"])
     nblocks = sum(m["blocks"] for m in desc["molecules"])
@@ -106,17 +115,19 @@ def recomputed_rows(N, ckpt):
 
 def grid_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     """Bytes one residual evaluation plus one DIIS update move on the grid
-    path, where every propagation step is a launch that streams its rows
-    through memory: forward 3w per site (read G(s-1) and G1, write G(s)),
-    backward with composition 6w (read Gb, G1 and Gf, write Gb, read and
-    write rho), 3w per recomputed row with checkpoints, over the interior
-    sites; the per-site arrays of the other phases and the DIIS history as
-    in hbm_bytes_per_evaluation."""
+    path, where a launch takes four propagation steps of every tile (the
+    tiles' halos come from the cache): forward the input row and G1 read once
+    per four steps and every row written, the same for the rows recomputed
+    with checkpoints; backward with composition Gb and G1 read, Gb written
+    and rho read and written per four steps and every Gf row read; over the
+    interior sites.  The per-site arrays of the other phases and the DIIS
+    history as in hbm_bytes_per_evaluation."""
     W = desc["MX"] * max(1, desc["MY"]) * max(1, desc["MZ"])
-    chains = sum((9 * m["chainlength"] + 3 * recomputed_rows(m["chainlength"], ckpt)) * w * W
-                 for m in desc["molecules"])
+    chains = sum(((2 / 4 + 1 + 5 / 4 + 1) * m["chainlength"] +
+                  (2 / 4 + 1) * recomputed_rows(m["chainlength"], ckpt)) * w * W
+                 for m in desc["molecules"] if m["chainlength"] > 1)
     rest = hbm_bytes_per_evaluation(desc, ckpt, w, kd) - \
-        sum(2 * w * m.get("size", 1) * W * stored_rows(m["chainlength"], ckpt) for m in desc["molecules"])
+        sum(end_point_bytes(desc, m, ckpt, w, W) for m in desc["molecules"])
     return chains + rest
 
 

@@ -81,7 +81,8 @@ typedef struct {
  * brackets, `(C)16(N)1[(N)1][(N)1](N)1`, dendrimers,
  * `@dend(A,(B)2,3; A,(B)2,3)` or `@dend(A,(B)6,3,(B)5(C)1,1)`, or combs,
  * `@comb((A)5; A,(B)3,(A)6,4; (A)7)` (the last three: first-order chains
- * without save_memory, run on the grid path); aliases, repeat groups and
+ * without save_memory; on a 1-gradient lattice whose rows fit LDS in one
+ * workgroup, else on the grid path); aliases, repeat groups and
  * @water are refused with SCF_E_PARSE and a message naming them.  Charged
  * systems (`mon : <name> : valence`, `epsilon`, `lat : <name> : bondlength`,
  * a molecule with freedom `neutralizer`) solve for the electrostatic

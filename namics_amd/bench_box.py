@@ -104,8 +104,8 @@ def run_box(args, n=96, seed=41):
         "mixed_precision": mixed,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "whole solve (per-kernel durations in profiles/k_step3_box96.md)",
+                     "kernel": "whole solve (per-kernel durations in profiles/k_box_box96.md)",
                      "bytes_per_solve": nbytes,
-                     "bytes": "every grid-path launch's streams: 9 x 8 B per site and contour step, 3 x 8 B per "
+                     "bytes": "every grid-path launch's streams: 3.75 x 8 B per site and contour step, 1.5 x 8 B per "
                               "recomputed row, per-site arrays once per evaluation, DIIS history per iteration"},
     }

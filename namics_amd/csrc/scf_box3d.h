@@ -19,7 +19,7 @@ namespace {
 // step 35 MB in 9.2 us, plus 2.5 us between launches; on 53^3 sites a step
 // took as long as its launch.  A tile reads row and weights once per kBoxH
 // steps, and the rows between two checkpoints are brought back by the launch
-// that composes them.  Chain of 20 segments, checkpoints every 5 rows: 381
+// that composes them.  Chain of 20 segments, checkpoints every 4 rows: 381
 // -> 230 us in 9 launches (from 48) on 96^3 sites, 53^3 sites 120 us.  What
 // is left is the halo: 15360 sites computed for 4608 owned (FP64 issue and
 // LDS about a third of a launch, its loads and start the rest).

@@ -905,7 +905,13 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
   auto consider = [&](int mode, int sx) {
     if (check_layout(S, mode, sx) == SCF_OK) cand.push_back({mode, sx});
   };
-  if (S->mode == SCF_MODE_AUTO && !markov2) consider(SCF_MODE_GRID, 0);
+  // (not the grid path's tiles where a 2-gradient chain has the strip or the
+  // register layout: alone they are a little faster, 64 x 128 layers, N = 200
+  // 0.59 for 0.67 ms per evaluation, but the choice holds for the shape, and
+  // queues and batches of it, many systems at once, need one workgroup each)
+  plan_layout(S, -1);
+  const bool resident = S->h.tile2 && (S->h.strip_sx > 0 || S->h.wave2 > 0);
+  if (S->mode == SCF_MODE_AUTO && !markov2 && !resident) consider(SCF_MODE_GRID, 0);
   if (S->mode != SCF_MODE_GRID) {
     if (l.gradients == 2) {
       for (int sx : {8, 4}) {

@@ -40,3 +40,24 @@ def test_checkpoint_intervals_equal_full_storage(mx, my):
         s.set_checkpoint(K)
         g, r = s.residual(x)
         assert r == want[1] and np.array_equal(g, want[0]), K
+
+
+@pytest.mark.gpu
+def test_tuned_shapes_still_batch():
+    """A shape whose layout was tuned on one system serves batches: the tuner
+    keeps one workgroup per system where a chain has such a layout."""
+    from namics_amd import ScfSystem, autotune_batch, autotune_forget
+    from namics_amd.workloads import brush_cylinder
+    autotune_forget()
+    try:
+        for nr, nz in ((64, 128), (43, 101)):
+            t = brush_cylinder(0.5, n_r=nr, n_z=nz, N=60)
+            s = ScfSystem(t)
+            s.autotune(evals=3)
+            assert s.layout()["mode"] == "fused"
+            s2 = ScfSystem(t)
+            autotune_batch([s, s2], evals=1)
+            s.close()
+            s2.close()
+    finally:
+        autotune_forget()

@@ -23,7 +23,7 @@ namespace {
 // -> 230 us in 9 launches (from 48) on 96^3 sites, 53^3 sites 120 us.  What
 // is left is the halo: 15360 sites computed for 4608 owned (FP64 issue and
 // LDS about a third of a launch, its loads and start the rest).
-constexpr int kBoxH = 4, kBoxZ = 32, kBoxOwnZ = kBoxZ - 2 * kBoxH;
+constexpr int kBoxZ = 32, kBoxOwnZ = kBoxZ - 2 * kBoxH;  // (kBoxH: scf_box_plan.h)
 constexpr int kBoxMaxWaves = 12;
 
 // What every launch of a chain needs of its system, in the kernel's own
@@ -46,26 +46,6 @@ __device__ __forceinline__ int box_layer(int p, int n, int periodic) {
   if (q < 0) q += period;
   return q < n ? q + 1 : 2 * n - q;
 }
-
-// Forward steps of a launch.
-struct BoxForward {
-  int n;            // steps
-  int src;          // slot of the input row; -1: the segment weight seg0
-  int seg0, slot0;  // slot0 >= 0: keep the input row there
-  int slot[kBoxH];  // end-point slot of each step's row, -1: not kept
-  int seg[kBoxH];
-};
-// Backward steps of a launch, after the forward steps that bring their rows.
-struct BoxRun {
-  BoxForward f;
-  int n;              // steps
-  int src;            // row of Gb to start from; -1: the segment weight seg0
-  int seg0, mm0;      // segment and density of the first row
-  int slot0;          // >= 0: compose the first row with it
-  int dst;            // row of Gb for the last row
-  int slot[kBoxH];    // end-point slot of each step's row
-  int seg[kBoxH], mm[kBoxH];
-};
 
 // Rows in FP64, or in FP32 with the molecule's gauge shift 
 // (G1' = G1 e^c, scf_grid.hip).  FP32 is what a row
@@ -331,90 +311,32 @@ hipError_t box_launch(const BoxShape &s, const BoxSys &S, const BoxForward *f, c
   }
 }
 
-// The chain of molecule mo in blocks of up to kBoxH rows.
+// The chain of molecule mo in launches of up to kBoxH rows.
 struct BoxChain {
-  const DevSys &h;
-  const int mo, N;
   const BoxShape shape;
-  const RowSlots loc;
-  std::vector<int> rb;  // block (segment, density) of every row
+  BoxSchedule plan;
   bool fp32;
   BoxSys S;
-  BoxChain(const DevSys &sys, int mol, bool f32)
-      : h(sys), mo(mol), N(sys.mol_N[mol]), shape(sys),
-        loc{sys.ckpt, sys.ckpt > 1 ? (N + sys.ckpt - 1) / sys.ckpt : N}, fp32(f32) {
-    for (int b = h.mol_block_begin[mo]; b < h.mol_block_begin[mo + 1]; b++) rb.insert(rb.end(), h.block_n[b], b);
+  BoxChain(const DevSys &h, int mo, bool f32) : shape(h), plan(h.mol_N[mo], h.ckpt), fp32(f32) {
+    for (int b = h.mol_block_begin[mo]; b < h.mol_block_begin[mo + 1]; b++) {
+      plan.seg.insert(plan.seg.end(), h.block_n[b], h.block_seg[b]);
+      plan.mm.insert(plan.mm.end(), h.block_n[b], h.block_mm[b]);
+    }
     const int own_y = 2 * shape.waves - 2 * kBoxH;
     S = {h.MX, h.MY, h.MZ, h.JX, h.JY,
          h.bx1 != 1, h.by1 != 1, h.bz1 != 1,
          (h.MY + own_y - 1) / own_y, (h.MZ + kBoxOwnZ - 1) / kBoxOwnZ, (size_t)h.M,
-         h.Gf, h.Gb, h.G1, h.rho, h.sc, mo, N};
+         h.Gf, h.Gb, h.G1, h.rho, h.sc, mo, h.mol_N[mo]};
   }
-  hipError_t launch(const BoxForward *f, const BoxRun *b, hipStream_t st) const {
-    return fp32 ? box_launch<float>(shape, S, f, b, st) : box_launch<double>(shape, S, f, b, st);
-  }
-  // Rows r0+1 .. r1 of the forward recursion from row r0; the last steps are
-  // left in `tail` for the backward launch that follows.  Of the first pass
-  // (`pass`) only the rows that outlive it are kept.
-  hipError_t forward(hipStream_t st, int r0, int r1, bool pass, BoxForward &tail) const {
-    const int K = h.ckpt;
-    for (int r = r0; r < r1;) {
-      BoxForward a{};
-      a.n = std::min(kBoxH, r1 - r);
-      a.src = r == 0 ? -1 : loc(r);
-      a.seg0 = h.block_seg[rb[0]];
-      a.slot0 = r == 0 ? loc(0) : -1;
-      for (int s = 0; s < a.n; s++) {
-        const int q = r + 1 + s;
-        const bool keep = !pass || K <= 1 || q % K == 0 || q / K == (N - 1) / K || s == a.n - 1;
-        a.slot[s] = keep ? loc(q) : -1;
-        a.seg[s] = h.block_seg[rb[q]];
-      }
-      r += a.n;
-      if (r == r1) {
-        tail = a;
-        break;
-      }
-      const hipError_t e = launch(&a, nullptr, st);
-      if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }
-  // The whole chain; gn() launches the sum over row N - 1 (slot loc(N - 1))
-  // while it is held.
+  // The whole chain; gn(slot) launches the sum over the last row while it is
+  // held there.
   template <typename Gn>
   hipError_t run(hipStream_t st, Gn gn) const {
-    const int K = h.ckpt;
-    int held = K > 1 ? (N - 1) / K : 0;  // the segment whose rows the buffer holds
-    int gb = 0;
-    for (int s = N - 1; s >= 0;) {
-      const bool first = s == N - 1;
-      BoxRun a{};
-      a.src = first ? -1 : gb;
-      a.seg0 = h.block_seg[rb[N - 1]];
-      a.mm0 = h.block_mm[rb[N - 1]];
-      a.slot0 = first ? loc(N - 1) : -1;
-      a.dst = gb = 1 - gb;
-      hipError_t e = hipSuccess;
-      if (first) {
-        e = forward(st, 0, N - 1, true, a.f);
-        s--;
-      } else if (K > 1 && s % K != 0 && s / K != held) {
-        held = s / K;
-        e = forward(st, held * K, held * K + K - 1, false, a.f);
-      }
-      if (e != hipSuccess) return e;
-      // rows as long as they are checkpoints or of the segment held
-      for (; a.n < kBoxH && s >= 0 && (K <= 1 || s % K == 0 || s / K == held); s--, a.n++) {
-        a.slot[a.n] = loc(s);
-        a.seg[a.n] = h.block_seg[rb[s]];
-        a.mm[a.n] = h.block_mm[rb[s]];
-      }
-      e = launch(nullptr, &a, st);
-      if (e != hipSuccess) return e;
-      if (first) gn();
-    }
-    return hipSuccess;
+    return (hipError_t)plan.run(
+        [&](const BoxForward *f, const BoxRun *b) -> int {
+          return fp32 ? box_launch<float>(shape, S, f, b, st) : box_launch<double>(shape, S, f, b, st);
+        },
+        [&] { gn(plan.loc(plan.N - 1)); });
   }
 };
 

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "scf_box_plan.h"
 #include "scf_device.h"
 #include "scf_kernels.h"
 #include "scf_spec.h"
@@ -654,26 +655,6 @@ __global__ void __launch_bounds__(kGridThreads) k_diis_combine_dev(const DevSys 
 }  // namespace nscf
 
 #include "scf_tile2d.h"
-
-namespace nscf {
-
-// End-point storage of the grid path.  With every row kept (ckpt <= 1) row
-// s of the forward recursion is Gf slot s.  With checkpoints every K rows
-// (the reference's save_memory, src/molecule.cpp:2300-2446) the slots hold
-// rows 0, K, 2K, ... (slot s/K) and one buffer of K-1 rows (slots nck ..
-// nck+K-2) for the rows between two checkpoints: the forward pass writes
-// each such row into the buffer, so after it the buffer holds the last
-// segment; the backward pass recomputes the rows of every earlier segment
-// from its checkpoint, with the forward arithmetic, just before it composes
-// them.  Densities and partition functions are bit-identical to full
-// storage.
-struct RowSlots {
-  int K, nck;
-  int operator()(int r) const { return K <= 1 ? r : (r % K == 0 ? r / K : nck + r % K - 1); }
-};
-
-}  // namespace nscf
-
 #include "scf_box3d.h"
 
 namespace nscf {
@@ -719,21 +700,21 @@ hipError_t grid_residual_body(const DevSys &h, DevSys *d, double *partial, int n
       chain.backward(d, st);
       continue;
     }
-    const RowSlots loc{h.ckpt, h.ckpt > 1 ? (N + h.ckpt - 1) / h.ckpt : N};
     if (six) {
       const BoxChain chain(h, mo, fp32);
-      const hipError_t e = chain.run(st, [&] {
+      const hipError_t e = chain.run(st, [&](int slot) {
         if (fp32) {
-          hipLaunchKernelGGL(k_gn_partial32, G, B, 0, st, d, loc(N - 1), partial);
+          hipLaunchKernelGGL(k_gn_partial32, G, B, 0, st, d, slot, partial);
           hipLaunchKernelGGL(k_finalize_gn32, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
         } else {
-          hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, loc(N - 1), partial);
+          hipLaunchKernelGGL(k_gn_partial, G, B, 0, st, d, slot, partial);
           hipLaunchKernelGGL(k_finalize_gn, dim3(1), dim3(kGridThreads), 0, st, d, partial, nb, mo);
         }
       });
       if (e != hipSuccess) return e;
       continue;
     }
+    const RowSlots loc{h.ckpt, h.ckpt > 1 ? (N + h.ckpt - 1) / h.ckpt : N};
     // block (segment, molecule-segment pair) of every row of the chain
     std::vector<int> rb;
     for (int b = b0; b < b1; b++) rb.insert(rb.end(), h.block_n[b], b);

@@ -100,11 +100,13 @@ struct scf_system {
   // Branched molecules on a 1-gradient lattice whose rows fit LDS run their
   // schedule in one workgroup (chain_branched) instead of one launch per row
   // operation, however many systems there are: 60 layers, 20 segments, about
-  // 100 operations: 0.27 -> 0.06 ms per evaluation.
+  // 100 operations: 0.27 -> 0.06 ms per evaluation.  Not with checkpoints (a
+  // linear molecule's save_memory): there the linear chains of one workgroup
+  // store every row, and the arena holds the checkpoints only.
   int mode_among(int n) const {
     const int m = effective_mode();
-    if (mode == SCF_MODE_AUTO && m == SCF_MODE_GRID && h.branch_lds && tuned_mode == SCF_MODE_AUTO &&
-        h.precision == SCF_PREC_FP64)
+    if (mode == SCF_MODE_AUTO && m == SCF_MODE_GRID && h.branch_lds && h.ckpt <= 1 &&
+        tuned_mode == SCF_MODE_AUTO && h.precision == SCF_PREC_FP64)
       return SCF_MODE_FUSED;
     const bool tiles = m == SCF_MODE_FUSED && mode == SCF_MODE_AUTO && tuned_mode == SCF_MODE_AUTO && h.tile2 &&
                        h.strip_sx == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;

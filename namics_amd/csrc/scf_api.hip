@@ -234,18 +234,19 @@ void plan_layout(scf_system *S, int want_sx) {
   }
   h.use_lds = rows <= lds_limit() ? 1 : 0;
   // branched molecules on 1-gradient lattices: their rows, the segment weights
-  // and the molecule's densities in LDS
+  // and the molecule's densities in LDS (the linear chains' rows fit or not
+  // by themselves: use_lds).  The linear molecules next to them are first
+  // order, as on the grid path.
+  size_t branch_bytes = 0;
   h.branch_lds = 0;
   if (l.gradients == 1 && S->branched()) {
-    size_t need = 0;
+    bool markov1 = true;
+    for (auto &m : S->spec.mol) markov1 = markov1 && m.markov == 1;
     for (size_t i = 0; i < S->plans.size(); i++)
       if (S->spec.mol[i].scheduled())
-        need = std::max(need, (size_t)(S->plans[i].rows + h.nseg + (int)S->spec.mol[i].molmon.size()) * M * D);
-    if (need <= lds_limit()) {
-      h.branch_lds = 1;
-      rows = std::max(h.use_lds ? rows : 0, need);
-      h.use_lds = 1;
-    }
+        branch_bytes = std::max(
+            branch_bytes, (size_t)(S->plans[i].rows + h.nseg + (int)S->spec.mol[i].molmon.size()) * M * D);
+    h.branch_lds = markov1 && branch_bytes <= lds_limit() ? 1 : 0;
   }
   // the lattice in registers, where its layers have lanes and its columns
   // waves; the generic chain stays selectable (want_sx = 0) next to a strip
@@ -265,7 +266,7 @@ void plan_layout(scf_system *S, int want_sx) {
       rows = std::max(h.strip_sx || rows <= lds_limit() ? rows : 0, edges + (h.wave2_own ? own : 0));
     }
   }
-  S->lds_bytes = h.use_lds ? rows : 0;
+  S->lds_bytes = std::max(h.use_lds ? rows : 0, h.branch_lds ? branch_bytes : 0);
 }
 
 // Layout choices the autotuner made, per lattice shape, for this process:

@@ -1,6 +1,6 @@
-"""Branched molecules next to linear ones on 1-gradient lattices, with the
-linear molecule's end points checkpointed: against the oracle, the grid path
-and full storage."""
+"""Branched molecules next to linear ones on 1-gradient lattices: the linear
+molecule's end points checkpointed, against the oracle and the grid path;
+second-order linear molecules, which the grid path refuses."""
 import numpy as np
 import pytest
 
@@ -65,3 +65,15 @@ def test_checkpointed_linear_molecule(fjc, how):
         got.append(g)
         s.close()
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,fjc", [(40, 1), (280, 4)])
+def test_second_order_linear_molecule_is_refused(layers, fjc):
+    """Also where the branched rows alone fit LDS and the linear ones (18 rows
+    of 1128 sites) do not."""
+    from namics_amd import ScfError, ScfSystem
+    s = ScfSystem(text(layers, 20, fjc, "mol : pol : Markov : 2\nmol : pol : k_stiff : 0.5\n"))
+    with pytest.raises(ScfError):
+        s.residual(np.zeros(s.nvar))
+    s.close()

@@ -171,7 +171,9 @@ int scf_system_set_graph(scf_system *sys, int on);
  * system's current device fields) for every layout that applies to the
  * lattice -- on 2-gradient lattices the register-strip widths SX = 8 and 4
  * and the generic site-strided chain; on 3-gradient lattices one workgroup
- * per system against one launch per phase -- keeps the fastest for this
+ * per system against one launch per phase; for branched molecules on a
+ * 1-gradient lattice their schedule in one workgroup against one launch per
+ * row operation -- keeps the fastest for this
  * system, and remembers it for the lattice shape, so systems built later in
  * the process with the same shape start from it.  Every layout computes the
  * same residual (to rounding).  A layout the system's options exclude (FP32

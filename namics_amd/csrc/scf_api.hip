@@ -285,7 +285,8 @@ std::string shape_key(const scf_system *S) {
   std::string k = std::to_string(l.gradients) + "/" + std::to_string(l.geometry) + "/" +
                   std::to_string(l.lattice_type) + "/" + std::to_string(l.MX) + "x" + std::to_string(l.MY) + "x" +
                   std::to_string(l.MZ) + "/f" + std::to_string(l.fjc);
-  for (auto &m : S->spec.mol) k += "/" + std::to_string(m.chainlength) + "m" + std::to_string(m.markov);
+  for (auto &m : S->spec.mol)
+    k += "/" + std::to_string(m.chainlength) + "m" + std::to_string(m.markov) + (m.scheduled() ? "b" : "");
   return k;
 }
 
@@ -920,6 +921,8 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
         if (S->h.strip_sx == sx) consider(SCF_MODE_FUSED, sx);
       }
       consider(SCF_MODE_FUSED, 0);
+    } else if (S->mode == SCF_MODE_AUTO && S->h.branch_lds && S->h.ckpt <= 1) {
+      cand.push_back({SCF_MODE_FUSED, 0});  // a branched schedule in one workgroup (mode_among)
     } else {
       consider(SCF_MODE_FUSED, 0);
     }
@@ -938,7 +941,7 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
     int rc = upload_solver(S);
     if (rc != SCF_OK) return rc;
     auto one = [&]() -> hipError_t {
-      if (S->effective_mode() == SCF_MODE_FUSED)
+      if (S->mode_among(1) == SCF_MODE_FUSED)
         return launch_fused(S->d_list, 1, FUSED_RESIDUAL, h.threads, S->lds_bytes, S->stream);
       hipError_t e = grid_residual(h, S->d, h.partial, S->nb, S->stream);
       return e != hipSuccess ? e : grid_thermo(h, S->d, h.partial, S->nb, S->stream);

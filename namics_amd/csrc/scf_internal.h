@@ -106,7 +106,7 @@ struct scf_system {
   int mode_among(int n) const {
     const int m = effective_mode();
     if (mode == SCF_MODE_AUTO && m == SCF_MODE_GRID && h.branch_lds && h.ckpt <= 1 &&
-        tuned_mode == SCF_MODE_AUTO && h.precision == SCF_PREC_FP64)
+        tuned_mode != SCF_MODE_GRID && h.precision == SCF_PREC_FP64)
       return SCF_MODE_FUSED;
     const bool tiles = m == SCF_MODE_FUSED && mode == SCF_MODE_AUTO && tuned_mode == SCF_MODE_AUTO && h.tile2 &&
                        h.strip_sx == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;

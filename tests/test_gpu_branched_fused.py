@@ -71,3 +71,30 @@ def test_batch_and_alone_agree():
     got, _ = solve_batch(b, xs)
     for s, x, y in zip(a, xs, got):
         assert np.array_equal(s.solve(x)[0], y)
+
+
+@pytest.mark.gpu
+def test_tuning_times_the_fused_schedule():
+    """The tuner has both routes of a branched system as candidates, and the
+    faster one, the fused one here, stays in use for systems of the shape
+    built later."""
+    from namics_amd import ScfSystem, autotune_forget, scf
+    autotune_forget()
+    t = with_layers(BRANCHED["branch1d_head"]["text"], 60)
+    try:
+        s = ScfSystem(t)
+        x = np.random.default_rng(2).uniform(-0.2, 0.2, s.nvar)
+        fused = s.residual(x)[0]
+        rep = s.autotune(evals=3)
+        print(rep, flush=True)
+        assert sorted(c["mode"] for c in rep["candidates"]) == ["fused", "grid"]
+        assert rep["candidates"][rep["chosen"]]["mode"] == "fused"
+        later = ScfSystem(t)
+        for k in (s, later):
+            assert np.array_equal(k.residual(x)[0], fused)
+            k.close()
+        grid = ScfSystem(t, mode=scf.MODE_GRID)  # an explicit mode leaves nothing to choose
+        assert grid.autotune(evals=1)["candidates"] == []
+        grid.close()
+    finally:
+        autotune_forget()

@@ -113,6 +113,133 @@ namespace nscf {
 // HBM; the row being read and the row being written live in LDS when they
 // fit.
 
+// 1-gradient Markov-1 chain that the wave tiles do not serve (a weight on a
+// surface ghost), one site per thread (M <= threads): the
+// neighbour indices and lattice weights of the site stay in registers for
+// the whole chain, and the density of a block is accumulated in a register.
+// LG1Planar::propagate (src/LG1Planar.cpp:146-149) and LGrad1::propagate
+// (src/LGrad1.cpp:441-445); a neighbour that falls on a ghost reads the site
+// set_bounds copies there, a missing neighbour (the stencil at the outermost
+// sites) has weight zero.  100 layers, N = 300: 179 us per evaluation, with the
+// site-strided chain 528.
+__device__ __noinline__ void chain1d_m1(const DevSys &S0, int mo) {
+  CSys &S = uniform_sys(S0);
+  const int M = S.M;
+  const int i = threadIdx.x;
+  const bool active = i < M;
+  const int ii = active ? i : 0;
+  const int i0 = map_x(S, ii);
+  const int im = ii >= 1 ? map_x(S, ii - 1) : i0;
+  const int ip = ii <= M - 2 ? map_x(S, ii + 1) : i0;
+  const bool planar = S.geometry == 0;
+  double wm, w0, wp;
+  if (planar) {
+    wm = S.lambda;
+    w0 = 1.0 - 2.0 * S.lambda;
+    wp = S.lambda;
+  } else {
+    wm = hbm(S.lam_m)[ii];
+    w0 = hbm(S.lam_0)[ii];
+    wp = hbm(S.lam_p)[ii];
+  }
+  if (ii < 1) wm = 0.0;
+  if (ii > M - 2) wp = 0.0;
+  const int b0 = S.mol_block_begin[mo], b1 = S.mol_block_begin[mo + 1];
+  const int N = S.mol_N[mo];
+  gdbl *Gf = hbm(S.Gf);
+  const gdbl *G1 = hbm(S.G1);
+  ldbl *ra = lds_row(0), *rb = lds_row(S.row_stride);
+
+  double g1 = active ? G1[(size_t)S.block_seg[b0] * M + ii] : 0.0;
+  double v = g1;
+  if (active) {
+    Gf[ii] = v;
+    ra[ii] = v;
+  }
+  lds_barrier();
+  ldbl *prev = ra, *next = rb;
+  int s = 1;
+  for (int b = b0; b < b1; b++) {
+    if (b != b0 && active) g1 = G1[(size_t)S.block_seg[b] * M + ii];
+    const int n = S.block_n[b] - (b == b0 ? 1 : 0);
+    for (int j = 0; j < n; j++, s++) {
+      if (active) {
+        double t;
+        if (planar) {
+          t = wm * prev[im];
+          t += w0 * prev[i0];
+        } else {
+          t = w0 * prev[i0];
+          t += wm * prev[im];
+        }
+        t += wp * prev[ip];
+        v = t * g1;
+        Gf[(size_t)s * M + ii] = v;
+        next[ii] = v;
+      }
+      lds_barrier();
+      ldbl *tmp = prev;
+      prev = next;
+      next = tmp;
+    }
+  }
+  // GN = weighted sum of the last end-point distribution (Lattice::ComputeGN)
+  {
+    double acc = 0.0;
+    if (active && ii >= 1 && ii <= S.MX) acc = (planar ? 1.0 : hbm(S.L)[ii]) * v;
+    const double gn = wg_sum(acc);
+    if (threadIdx.x == 0) S0.sc->GN[mo] = gn;
+  }
+  // backward with composition, Gf(s-1) fetched one step ahead.  On a ghost
+  // the composition reads Gf(s) as the reference leaves it: the value
+  // set_bounds copied there when Gf(s) propagated to s+1 (the site i0), and
+  // zero for the last row, whose ghosts ComputeGN's remove_bounds cleared
+  // (src/LGrad1.cpp:213-221,863-874).  Only phitot on the ghosts sees this.
+  ldbl *ga = ra, *gb = rb;
+  const int bl = b1 - 1;
+  const bool ghost = ii < 1 || ii > S.MX;
+  g1 = active ? G1[(size_t)S.block_seg[bl] * M + ii] : 0.0;
+  v = g1;
+  double racc = 0.0, gf = 0.0;
+  if (active) {
+    racc = (ghost ? 0.0 : Gf[(size_t)(N - 1) * M + ii]) * v;
+    ga[ii] = v;
+    if (N >= 2) gf = Gf[(size_t)(N - 2) * M + i0];
+  }
+  lds_barrier();
+  s = N - 2;
+  for (int b = bl; b >= b0; b--) {
+    if (b != bl) {
+      if (active) g1 = G1[(size_t)S.block_seg[b] * M + ii];
+      racc = 0.0;
+    }
+    const int n = S.block_n[b] - (b == bl ? 1 : 0);
+    for (int j = 0; j < n; j++, s--) {
+      if (active) {
+        double t;
+        if (planar) {
+          t = wm * ga[im];
+          t += w0 * ga[i0];
+        } else {
+          t = w0 * ga[i0];
+          t += wm * ga[im];
+        }
+        t += wp * ga[ip];
+        v = t * g1;
+        racc += gf * v;
+        gb[ii] = v;
+        if (s >= 1) gf = Gf[(size_t)(s - 1) * M + i0];
+      }
+      lds_barrier();
+      ldbl *tmp = ga;
+      ga = gb;
+      gb = tmp;
+    }
+    if (active) hbm(S.rho)[(size_t)S.block_mm[b] * M + ii] += racc;
+  }
+  __syncthreads();
+}
+
 // Ring of a first-order chain on a 1-gradient lattice (fjc = 1), one site
 // per thread (mol_linear::ComputePhi src/mol_linear.cpp:35-111).  The first
 // and last blocks are one segment each of the same type, merged: for every
@@ -219,6 +346,167 @@ __device__ __noinline__ void chain1d_ring(const DevSys &S0, int mo) {
   if (active) hbm(S.rho)[(size_t)S.block_mm[b0] * M + ii] += racc_a;
   const double gn = wg_sum(gnacc);
   if (threadIdx.x == 0) S0.sc->GN[mo] = gn;
+  __syncthreads();
+}
+
+// Second-order (Markov 2) chain on a 1-gradient simple-cubic lattice that the
+// wave tiles do not serve (periodic, more waves than a workgroup has, a weight
+// on a surface ghost), one site per thread (M <= threads), rows in LDS: three direction components per
+// site (+x, lateral, -x), the stencil of m2_step, composition weights
+// (1/6, 4/6, 1/6) (LGrad1::AddPhiS src/LGrad1.cpp:876-910),
+// GN = (G0 + 4 G1 + G2) / 6 (LGrad1::ComputeGN src/LGrad1.cpp:943-955).
+// The arithmetic is chain_markov2's, in the same order; what differs is that
+// no global access sits on a step's critical path: the Boltzmann weight of a
+// block and its density stay in registers (the density is read once at the
+// block's start and written once at its end), and Gf of the backward pass is
+// fetched one step ahead.  N = 500, per evaluation: 100 periodic layers 0.90
+// ms, with the site-strided chain 1.23; 950 layers 1.46 and 2.21.
+template <int kSPT>
+__device__ __noinline__ void chain1d_m2(const DevSys &S0, int mo) {
+  CSys &S = uniform_sys(S0);
+  const int M = S.M;
+  const int tid = work_tid(S), nt = S.threads;
+  const int R = 3 * M;
+  double P[kMaxComp];
+#pragma unroll
+  for (int k = 0; k < kMaxComp; k++) P[k] = S.mol_P[mo][k];
+  constexpr double wc[3] = {1.0 / 6.0, 4.0 / 6.0, 1.0 / 6.0};
+  int ii[kSPT];
+  bool act[kSPT];
+#pragma unroll
+  for (int k = 0; k < kSPT; k++) {
+    const int w = tid + k * nt;
+    act[k] = w < M;
+    ii[k] = act[k] ? w : 0;
+  }
+  const int b0 = S.mol_block_begin[mo], b1 = S.mol_block_begin[mo + 1];
+  const int N = S.mol_N[mo];
+  gdbl *Gf = hbm(S.Gf);
+  const gdbl *G1 = hbm(S.G1);
+  ldbl *ra = lds_row(0), *rb = lds_row(S.row_stride);
+  double g1[kSPT], o[kSPT][3];
+#pragma unroll
+  for (int k = 0; k < kSPT; k++) {
+    g1[k] = act[k] ? G1[(size_t)S.block_seg[b0] * M + ii[k]] : 0.0;
+    if (act[k])
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        Gf[c * M + ii[k]] = g1[k];
+        ra[c * M + ii[k]] = g1[k];
+      }
+  }
+  lds_barrier();
+  ldbl *prev = ra, *next = rb;
+  int s = 1;
+  for (int b = b0; b < b1; b++) {
+    if (b != b0) {
+#pragma unroll
+      for (int k = 0; k < kSPT; k++)
+        if (act[k]) g1[k] = G1[(size_t)S.block_seg[b] * M + ii[k]];
+    }
+    for (int j = (b == b0 ? 1 : 0); j < S.block_n[b]; j++, s++) {
+#pragma unroll
+      for (int k = 0; k < kSPT; k++) {
+        m2_step<double>(S, (const ldbl *)prev, P, true, ii[k], o[k]);
+#pragma unroll
+        for (int c = 0; c < 3; c++) o[k][c] *= g1[k];
+      }
+      gdbl *gs = Gf + (size_t)s * R;
+#pragma unroll
+      for (int k = 0; k < kSPT; k++)
+        if (act[k])
+#pragma unroll
+          for (int c = 0; c < 3; c++) {
+            gs[c * M + ii[k]] = o[k][c];
+            next[c * M + ii[k]] = o[k][c];
+          }
+      lds_barrier();
+      ldbl *t = prev;
+      prev = next;
+      next = t;
+    }
+  }
+  {
+    double a[3] = {0.0, 0.0, 0.0};
+    const gdbl *gl = Gf + (size_t)(N - 1) * R;
+#pragma unroll
+    for (int k = 0; k < kSPT; k++)
+      if (act[k] && ii[k] >= 1 && ii[k] <= S.MX) {
+        const double wt = site_weight(S0, ii[k]);
+#pragma unroll
+        for (int c = 0; c < 3; c++) a[c] += wt * gl[c * M + ii[k]];
+      }
+    double gn = wg_sum(a[0]);
+    gn += 4.0 * wg_sum(a[1]);
+    gn += wg_sum(a[2]);
+    if (threadIdx.x == 0) S0.sc->GN[mo] = gn / 6.0;
+  }
+  // backward with composition; Gf(s) of every component fetched one step
+  // ahead, the block density in registers
+  ldbl *gbA = ra, *gbB = rb;
+  const int bl = b1 - 1;
+  double racc[kSPT], gf[kSPT][3];
+  {
+    const gdbl *gfl = Gf + (size_t)(N - 1) * R;
+#pragma unroll
+    for (int k = 0; k < kSPT; k++) {
+      g1[k] = act[k] ? G1[(size_t)S.block_seg[bl] * M + ii[k]] : 0.0;
+      racc[k] = act[k] ? hbm(S.rho)[(size_t)S.block_mm[bl] * M + ii[k]] : 0.0;
+      // ghosts: the last row reads zero (ComputeGN's remove_bounds), earlier
+      // rows the components set_bounds(X, Y) paired there (m2_val)
+      const bool ghost = ii[k] < 1 || ii[k] > S.MX;
+      if (act[k]) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          gbA[c * M + ii[k]] = g1[k];
+          racc[k] += wc[c] * (ghost ? 0.0 : gfl[c * M + ii[k]]) * g1[k];
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        gf[k][c] = (act[k] && N >= 2) ? m2_val<double>(S, Gf + (size_t)(N - 2) * R, c, ii[k]) : 0.0;
+    }
+  }
+  lds_barrier();
+  s = N - 2;
+  for (int b = bl; b >= b0; b--) {
+    if (b != bl) {
+#pragma unroll
+      for (int k = 0; k < kSPT; k++) {
+        if (act[k]) {
+          hbm(S.rho)[(size_t)S.block_mm[b + 1] * M + ii[k]] = racc[k];
+          g1[k] = G1[(size_t)S.block_seg[b] * M + ii[k]];
+          racc[k] = hbm(S.rho)[(size_t)S.block_mm[b] * M + ii[k]];
+        }
+      }
+    }
+    for (int j = (b == bl ? S.block_n[b] - 2 : S.block_n[b] - 1); j >= 0; j--, s--) {
+#pragma unroll
+      for (int k = 0; k < kSPT; k++) {
+        m2_step<double>(S, (const ldbl *)gbA, P, false, ii[k], o[k]);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          o[k][c] *= g1[k];
+          racc[k] += wc[c] * gf[k][c] * o[k][c];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kSPT; k++)
+        if (act[k])
+#pragma unroll
+          for (int c = 0; c < 3; c++) {
+            gbB[c * M + ii[k]] = o[k][c];
+            if (s >= 1) gf[k][c] = m2_val<double>(S, Gf + (size_t)(s - 1) * R, c, ii[k]);
+          }
+      lds_barrier();
+      ldbl *t = gbA;
+      gbA = gbB;
+      gbB = t;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kSPT; k++)
+    if (act[k]) hbm(S.rho)[(size_t)S.block_mm[b0] * M + ii[k]] = racc[k];
   __syncthreads();
 }
 
@@ -1892,7 +2180,9 @@ __device__ double fused_residual(const DevSys &S0) {
             chain1d_tile<3, false>(S0, mo);
           else
             chain1d_tile<3, true>(S0, mo);
-        } else if (kind == M2_SC1)
+        } else if (kind == M2_SC1 && S.M <= S.threads)
+          chain1d_m2<1>(S0, mo);
+        else if (kind == M2_SC1)
           chain_markov2<true, M2_SC1>(S0, mo);
         else if (kind == M2_HEX1)
           chain_markov2<true, M2_HEX1>(S0, mo);
@@ -1928,6 +2218,8 @@ __device__ double fused_residual(const DevSys &S0) {
         chain1d_tile<1, false>(S0, mo);
       else
         chain1d_tile<1, true>(S0, mo);
+    } else if (S.gradients == 1 && S.fjc == 1 && S.use_lds && S.M <= S.threads) {
+      chain1d_m1(S0, mo);
     } else if (S.use_lds) {
       chain_markov1<true>(S0, mo);
     } else {

@@ -11,9 +11,18 @@
 #include "scf_kernels.h"
 #include "scf_spec.h"
 
-// Sites per system and system of a call above which 2-gradient tiles are
-// faster (scf_system::mode_among).
-constexpr int kTileSites = 640;
+// 2-gradient tiles are faster while a call has no more systems than the
+// lattice has 700 + 24000 / N sites (scf_system::mode_among; N segments in
+// all its chains): tiles take one system after another, 2.5 us per segment and
+// a fixed part for launches and the passes around the chains.  Batches of n
+// solves of 3 evaluations, one workgroup each against tiles, ms:
+//   100 x 100, N = 8     n = 3   2.5   1.8   n = 5   3.0   3.0
+//   100 x 100, N = 20    n = 5   4.3   3.6   n = 7   4.8   5.0
+//   128 x 256, N = 20    n = 16 18.7  16.4   n = 24 23.9  24.6
+//   97 x 102, N = 100    n = 8  13.8  10.3   n = 12 14.9  15.4
+//   128 x 256, N = 100   n = 32 69.8  61.1   n = 45 63.7  68.2
+//   128 x 200, N = 400   n = 30 152   118    n = 40 145   144
+constexpr int kTileSites = 700, kTileFixed = 24000;
 
 // One SCF system: its parsed input, device description and HBM arena.
 struct scf_system {
@@ -89,9 +98,9 @@ struct scf_system {
   // 2-gradient lattice whose rows do not fit LDS (from about 9800 sites off
   // the strip path) runs its chains as tiles over many workgroups
   // (scf_tile2d.h) while the call is small: one after another, such systems
-  // take about 2.5 us per contour index each, while one launch of a workgroup
-  // per system takes 4 ns per site and contour index whatever their number up
-  // to one per CU.  Alone, per evaluation: 101 x 128, N = 100: 5.14 -> 0.38
+  // take the time of their launches each, while one launch of a workgroup per
+  // system takes 4 ns per site and contour index whatever their number up to
+  // one per CU.  Alone, per evaluation: 101 x 128, N = 100: 5.14 -> 0.38
   // ms; 128 x 256, N = 400: 49.5 -> 1.09 ms.  Lattices with their rows in LDS
   // stay with one workgroup each: tiles would be 1.4 to 4 times faster alone,
   // but a served or batched system gives the bits it gives alone, and there
@@ -110,7 +119,10 @@ struct scf_system {
       return SCF_MODE_FUSED;
     const bool tiles = m == SCF_MODE_FUSED && mode == SCF_MODE_AUTO && tuned_mode == SCF_MODE_AUTO && h.tile2 &&
                        h.strip_sx == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;
-    return tiles && (long long)n * kTileSites <= (long long)spec.lat.MX * spec.lat.MY ? SCF_MODE_GRID : m;
+    if (!tiles) return m;
+    long long N = 0;
+    for (auto &mol : spec.mol) N += mol.chainlength;
+    return n * (kTileSites * N + kTileFixed) <= N * spec.lat.MX * spec.lat.MY ? SCF_MODE_GRID : m;
   }
 };
 

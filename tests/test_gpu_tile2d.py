@@ -83,3 +83,20 @@ def test_large_lattices_take_the_tiles_alone(save_memory):
     for s in (a, b):
         s.set_solver(iterationlimit=5)
     assert np.array_equal(a.solve(x)[0], b.solve(x)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,tiles", [(2, True), (5, True), (6, False), (12, False)])
+def test_batches_change_to_one_workgroup_each(n, tiles):
+    """97 x 102 layers, 24 segments: up to five systems of a call run as tiles,
+    more in one launch of a workgroup each."""
+    from namics_amd import ScfSystem, scf, solve_batch
+    t = text(97, 102, "(A)12(B)11", "planar", "simple_cubic", "") + "newton : isaac : iterationlimit : 2\n"
+    alone = ScfSystem(t, mode=scf.MODE_GRID if tiles else scf.MODE_FUSED)
+    systems = [ScfSystem(t) for _ in range(n)]
+    xs = [np.random.default_rng(i).uniform(-0.1, 0.1, alone.nvar) for i in range(n)]
+    got, _ = solve_batch(systems, xs)
+    for x, y in zip(xs, got):
+        assert np.array_equal(alone.solve(x)[0], y)
+    for s in systems + [alone]:
+        s.close()

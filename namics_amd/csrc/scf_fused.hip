@@ -2210,7 +2210,7 @@ __device__ double fused_residual(const DevSys &S0) {
     } else if (S.all_sites) {
       chain_literal(S0, mo);
     } else if (S.wave2 > 0 && !fp32) {
-      chain_wave2_select(S0, mo);
+      chain_wave2(S0, mo);
     } else if (S.strip_sx > 0) {
       chain_strip_dispatch(S0, mo, fp32, fp32 ? sc.lnshift[mo] : 0.0);
     } else if (tile_serves(S, mo)) {

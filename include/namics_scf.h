@@ -169,13 +169,13 @@ int scf_system_set_graph(scf_system *sys, int on);
 
 /* Launch-layout autotuner.  Times `evals` residual evaluations (at the
  * system's current device fields) for every layout that applies to the
- * lattice -- on 2-gradient lattices the register-strip widths SX = 8 and 4
- * and the generic site-strided chain; on 3-gradient lattices one workgroup
- * per system against one launch per phase; for branched molecules on a
- * 1-gradient lattice their schedule in one workgroup against one launch per
- * row operation -- keeps the fastest for this
- * system, and remembers it for the lattice shape, so systems built later in
- * the process with the same shape start from it.  Every layout computes the
+ * lattice -- on 2-gradient lattices the whole lattice in registers, the
+ * register-strip widths SX = 8 and 4 and the generic site-strided chain; on
+ * 3-gradient lattices one workgroup per system against one launch per phase;
+ * for branched molecules on a 1-gradient lattice their schedule in one
+ * workgroup against one launch per row operation -- keeps the fastest for
+ * this system, and remembers it for the lattice shape, so systems built later
+ * in the process with the same shape start from it.  Every layout computes the
  * same residual (to rounding).  A layout the system's options exclude (FP32
  * propagators need a strip layout, checkpointing a strip layout or the grid
  * path; an explicit scf_system_set_mode) is not tried.  No counterpart in the reference, which
@@ -185,7 +185,8 @@ typedef struct {
   int candidates;                   /* layouts timed */
   int chosen;                       /* index of the fastest */
   int mode[SCF_TUNE_MAX];           /* SCF_MODE_FUSED / SCF_MODE_GRID */
-  int strip_sx[SCF_TUNE_MAX];       /* fused path: 8, 4, or 0 for the generic chain */
+  int strip_sx[SCF_TUNE_MAX];       /* fused path: 8, 4, or 0 off the strips; the lattice in registers
+                                       comes first, with the strip width of its FP32 chains */
   double ms_per_eval[SCF_TUNE_MAX]; /* device time of one residual evaluation */
 } scf_tune_report;
 int scf_system_autotune(scf_system *sys, int evals, scf_tune_report *report);

@@ -190,11 +190,26 @@ double fraction(const MoleculeSpec &m, int seg) {
 }
 
 // ---------------------------------------------------------------- layouts
+// Whether the chains of a 2-gradient lattice run faster in registers than in
+// strips of width sx (the first that fits), for MY layers along the lanes.
+// Registers pay by the lane, used or not (64, 128 or 256 layers of them), a
+// strip by the layer, and strips of 4 have twice the threads for a small
+// lattice.  Time in strips over time in registers, one residual evaluation,
+// N = 200, MX 32 .. 128 (a row each where it fits):
+//   strips of 8   MY 32 0.76-0.83, 48 0.88-0.94, 60 0.94-1.05, 64 1.04-1.14,
+//                 65-76 0.95-1.07, 80 0.99-1.07, 84 1.01-1.11, 96 1.03-1.14,
+//                 128 1.28-1.33, 129 1.03, 192 1.14, 256 1.21
+//   strips of 4   MY 32 0.60-0.70, 64 0.78-0.89, 96 0.96, 112 0.99
+// 256 systems at once are up to a tenth faster in registers at 65 to 80 layers.
+bool registers_faster(int sx, int MY) { return sx == 8 && (MY == 64 || MY >= 84); }
+
 // Launch layout of the fused path: threads per system, whether the
 // propagator rows live in LDS, and on 2-gradient lattices the register-strip
 // width SX (8 or 4 sites per thread along x; 0 = the generic site-strided
-// chain).  want_sx < 0 picks the first strip width that fits.
-void plan_layout(scf_system *S, int want_sx) {
+// chain).  want_sx < 0 picks the first strip width that fits.  registers: 1
+// keeps 2-gradient lattices in registers (scf_chain2d.h) wherever they fit,
+// next to a strip layout for FP32 chains; 0 nowhere; -1 where it is faster.
+void plan_layout(scf_system *S, int want_sx, int registers) {
   const LatticeSpec &l = S->spec.lat;
   DevSys &h = S->h;
   const size_t D = sizeof(double);
@@ -249,32 +264,30 @@ void plan_layout(scf_system *S, int want_sx) {
     h.branch_lds = markov1 && branch_bytes <= lds_limit() ? 1 : 0;
   }
   // the lattice in registers, where its layers have lanes and its columns
-  // waves; the generic chain stays selectable (want_sx = 0) next to a strip
-  // layout
+  // waves
+  size_t wave2_bytes = 0;
   h.wave2 = h.wave2_own = 0;
-  bool strip_possible = false;
-  for (int sx : {8, 4}) strip_possible = strip_possible || (strip_ok && l.MX % sx == 0 && (l.MX / sx) * l.MY <= 1024);
-  const int yp = strip_ok && (want_sx != 0 || !strip_possible) ? wave2_layers(l.MY) : 0;
+  const int yp = strip_ok && registers != 0 ? wave2_layers(l.MY) : 0;
   if (yp > 0) {
     const int nw = (l.MX + kWave2Sites / yp - 1) / (kWave2Sites / yp);
     const size_t edges = (size_t)2 * nw * 128 * yp * D, own = (size_t)1024 * kWave2Sites * D;
-    if (nw <= 16 && edges <= lds_limit()) {
+    if (nw <= 16 && edges <= lds_limit() && (registers == 1 || h.strip_sx == 0 || registers_faster(h.strip_sx, l.MY))) {
       h.wave2 = yp;
       h.wave2_own = edges + own <= lds_limit() ? 1 : 0;
       h.threads = std::max(h.threads, 64 * nw);
-      h.use_lds = 1;
-      rows = std::max(h.strip_sx || rows <= lds_limit() ? rows : 0, edges + (h.wave2_own ? own : 0));
+      wave2_bytes = edges + (h.wave2_own ? own : 0);
     }
   }
-  S->lds_bytes = std::max(h.use_lds ? rows : 0, h.branch_lds ? branch_bytes : 0);
+  S->lds_bytes = std::max({h.use_lds ? rows : 0, h.branch_lds ? branch_bytes : 0, wave2_bytes});
 }
 
 // Layout choices the autotuner made, per lattice shape, for this process:
 // systems built later with the same shape start from the tuned layout.
 namespace {
 struct TunedLayout {
-  int mode;      // SCF_MODE_FUSED or SCF_MODE_GRID
-  int strip_sx;  // fused path: 8, 4 or 0
+  int mode;       // SCF_MODE_FUSED or SCF_MODE_GRID
+  int strip_sx;   // fused path: 8, 4 or 0
+  int registers;  // 2 gradients: the lattice in registers
 };
 std::mutex g_tune_mu;
 std::map<std::string, TunedLayout> g_tuned;
@@ -290,12 +303,15 @@ std::string shape_key(const scf_system *S) {
   return k;
 }
 
-int tuned_strip(scf_system *S) {
-  std::lock_guard<std::mutex> lk(g_tune_mu);
-  auto it = g_tuned.find(shape_key(S));
-  if (it == g_tuned.end()) return -1;
-  S->tuned_mode = it->second.mode;
-  return it->second.strip_sx;
+void plan_tuned(scf_system *S) {
+  TunedLayout t{SCF_MODE_AUTO, -1, -1};
+  {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    auto it = g_tuned.find(shape_key(S));
+    if (it != g_tuned.end()) t = it->second;
+  }
+  S->tuned_mode = t.mode;
+  plan_layout(S, t.strip_sx, t.registers);
 }
 
 int build(scf_system *S, const Placement *pl) {
@@ -615,7 +631,7 @@ int build(scf_system *S, const Placement *pl) {
   h.x0 = P(o_x0);
   h.sc = (DevScalars *)(base + o_sc);
   h.partial = P(o_part);
-  plan_layout(S, tuned_strip(S));
+  plan_tuned(S);
   h.precision = SCF_PREC_FP64;
   h.mixed_switch = 1e-4;
   {
@@ -904,40 +920,44 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
   bool markov2 = false;
   for (auto &m : S->spec.mol) markov2 = markov2 || m.markov == 2;
   std::vector<TunedLayout> cand;
-  auto consider = [&](int mode, int sx) {
-    if (check_layout(S, mode, sx) == SCF_OK) cand.push_back({mode, sx});
+  auto consider = [&](int mode, int sx, int registers) {
+    if (check_layout(S, mode, sx) == SCF_OK) cand.push_back({mode, sx, registers});
   };
   // (not the grid path's tiles where a 2-gradient chain has the strip or the
   // register layout: alone they are a little faster, 64 x 128 layers, N = 200
   // 0.59 for 0.67 ms per evaluation, but the choice holds for the shape, and
   // queues and batches of it, many systems at once, need one workgroup each)
-  plan_layout(S, -1);
+  plan_layout(S, -1, 1);
   const bool resident = S->h.tile2 && (S->h.strip_sx > 0 || S->h.wave2 > 0);
-  if (S->mode == SCF_MODE_AUTO && !markov2 && !resident) consider(SCF_MODE_GRID, 0);
+  if (S->mode == SCF_MODE_AUTO && !markov2 && !resident) consider(SCF_MODE_GRID, 0, 0);
   if (S->mode != SCF_MODE_GRID) {
     if (l.gradients == 2) {
+      if (S->h.wave2 > 0) consider(SCF_MODE_FUSED, S->h.strip_sx, 1);
       for (int sx : {8, 4}) {
-        plan_layout(S, sx);
-        if (S->h.strip_sx == sx) consider(SCF_MODE_FUSED, sx);
+        plan_layout(S, sx, 0);
+        if (S->h.strip_sx == sx) consider(SCF_MODE_FUSED, sx, 0);
       }
-      consider(SCF_MODE_FUSED, 0);
+      consider(SCF_MODE_FUSED, 0, 0);
     } else if (S->mode == SCF_MODE_AUTO && S->h.branch_lds && S->h.ckpt <= 1) {
-      cand.push_back({SCF_MODE_FUSED, 0});  // a branched schedule in one workgroup (mode_among)
+      cand.push_back({SCF_MODE_FUSED, 0, 0});  // a branched schedule in one workgroup (mode_among)
     } else {
-      consider(SCF_MODE_FUSED, 0);
+      consider(SCF_MODE_FUSED, 0, 0);
     }
   }
   if (cand.empty()) {
-    plan_layout(S, -1);
+    plan_layout(S, -1, -1);
     return check_layout(S, S->effective_mode(), S->h.strip_sx);
   }
   const int saved_mode = S->mode, saved_tuned = S->tuned_mode;
   double best = 1e300;
   int besti = 0;
   DevSys &h = S->h;
+  auto plan = [&](const TunedLayout &t) {
+    plan_layout(S, t.mode == SCF_MODE_FUSED && l.gradients == 2 ? t.strip_sx : -1, t.registers);
+  };
   for (size_t c = 0; c < cand.size() && c < SCF_TUNE_MAX; c++) {
     S->tuned_mode = cand[c].mode;
-    plan_layout(S, cand[c].mode == SCF_MODE_FUSED && l.gradients == 2 ? cand[c].strip_sx : -1);
+    plan(cand[c]);
     int rc = upload_solver(S);
     if (rc != SCF_OK) return rc;
     auto one = [&]() -> hipError_t {
@@ -972,10 +992,10 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
     }
   }
   rep->chosen = besti;
-  TunedLayout pick{rep->mode[besti], rep->strip_sx[besti]};
+  const TunedLayout pick = cand[besti];
   S->mode = saved_mode;
   S->tuned_mode = saved_mode == SCF_MODE_AUTO ? pick.mode : saved_tuned;
-  plan_layout(S, pick.mode == SCF_MODE_FUSED && l.gradients == 2 ? pick.strip_sx : -1);
+  plan(pick);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[shape_key(S)] = pick;
@@ -1004,19 +1024,22 @@ int scf_autotune_batch(scf_system *const *systems, int n, int evals, scf_batch_t
   }
   // end-point storages every system can hold (the input's save_memory sizes
   // the arena for checkpoints only)
-  // (interval 3 only where the rows of interval 2 outgrow the 256 MB
-  // last-level cache: 256 brushes of 64 x 128 layers, N = 200, 1.29 -> 1.21 ms
-  // per evaluation; within the cache it only adds steps)
+  // (interval 3 only for chains in registers, where it is on chip, and where
+  // the rows of interval 2 outgrow the 256 MB last-level cache: 256 brushes of
+  // 64 x 128 layers, N = 200, 1.29 -> 1.21 ms per evaluation; within the cache
+  // it only adds steps)
   std::vector<int> cand;
+  bool registers = true;
   double kept = 0;  // bytes of the rows of interval 2
   for (int i = 0; i < n; i++) {
     int rows = 0;
     for (auto &m : systems[i]->spec.mol) rows = std::max(rows, ckpt_rows(m.chainlength, 2) * m.size);
     kept += (double)rows * systems[i]->spec.lat.M * sizeof(double);
+    registers = registers && systems[i]->h.wave2 > 0;
   }
   for (int K : {1, 2, 3}) {
     bool fits = K == 1 || strip;
-    if (K == 3 && kept < 256e6) continue;
+    if (K == 3 && !(registers && kept >= 256e6)) continue;
     for (int i = 0; i < n && fits; i++)
       for (auto &m : systems[i]->spec.mol) fits = fits && ckpt_rows(m.chainlength, K) * m.size <= systems[i]->gf_rows;
     if (fits) cand.push_back(K);

@@ -10,7 +10,8 @@ namespace nscf {
 // lane itself or the adjacent lanes (DPP) and only the column sums of a
 // wave's two outer columns go through LDS: 64 bytes per thread and step with
 // one barrier, where keeping the row in LDS moved 240 (64 x 128 layers: 1.7
-// us per step, bound by that traffic).  Any number of layers fits that has
+// us per step, bound by that traffic; strips remain for the FP32 chains and for
+// shapes that leave too many lanes idle, registers_faster in scf_api.hip).  Any number of layers fits that has
 // the lanes and waves: MY <= 64 YP, MX <= 16 SX.  (kFull: every lane and
 // column is inside the lattice.)
 //

@@ -118,7 +118,7 @@ struct scf_system {
         tuned_mode != SCF_MODE_GRID && h.precision == SCF_PREC_FP64)
       return SCF_MODE_FUSED;
     const bool tiles = m == SCF_MODE_FUSED && mode == SCF_MODE_AUTO && tuned_mode == SCF_MODE_AUTO && h.tile2 &&
-                       h.strip_sx == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;
+                       h.strip_sx == 0 && h.wave2 == 0 && !h.use_lds && h.precision == SCF_PREC_FP64;
     if (!tiles) return m;
     long long N = 0;
     for (auto &mol : spec.mol) N += mol.chainlength;
@@ -159,8 +159,8 @@ int lbfgs_solve(scf_system *S, scf_solve_info *info);
 int brr_solve(scf_system *S, scf_solve_info *info);
 double wall_clock_khz();
 size_t lds_limit();
-void plan_layout(scf_system *S, int want_sx);
-int tuned_strip(scf_system *S);
+void plan_layout(scf_system *S, int want_sx, int registers);
+void plan_tuned(scf_system *S);
 std::string shape_key(const scf_system *S);
 // End-point rows kept with checkpoint interval K (K <= 1: all N rows): the
 // checkpoints 0, K, 2K, ... plus a buffer for the rows of one segment.

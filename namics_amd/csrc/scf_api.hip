@@ -944,6 +944,10 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
       consider(SCF_MODE_FUSED, 0, 0);
     }
   }
+  // ... unless the options leave nothing else (checkpoints off the strips,
+  // branched molecules): timed, but no choice to remember for the shape
+  const bool only_grid = cand.empty() && S->mode == SCF_MODE_AUTO && !markov2;
+  if (only_grid) consider(SCF_MODE_GRID, -1, -1);
   if (cand.empty()) {
     plan_layout(S, -1, -1);
     return check_layout(S, S->effective_mode(), S->h.strip_sx);
@@ -994,9 +998,9 @@ int scf_system_autotune(scf_system *S, int evals, scf_tune_report *rep) {
   rep->chosen = besti;
   const TunedLayout pick = cand[besti];
   S->mode = saved_mode;
-  S->tuned_mode = saved_mode == SCF_MODE_AUTO ? pick.mode : saved_tuned;
+  S->tuned_mode = saved_mode == SCF_MODE_AUTO && !only_grid ? pick.mode : saved_tuned;
   plan(pick);
-  {
+  if (!only_grid) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[shape_key(S)] = pick;
   }

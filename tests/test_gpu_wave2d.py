@@ -61,3 +61,27 @@ def test_tuned_shapes_still_batch():
             s2.close()
     finally:
         autotune_forget()
+
+
+@pytest.mark.gpu
+def test_tuner_times_the_grid_path_where_nothing_else_runs():
+    """Checkpoints off the strips and branched molecules run on the grid path
+    alone: the one candidate, which is not remembered for the shape."""
+    from namics_amd import ScfSystem, autotune_batch, autotune_forget
+    from namics_amd.workloads import brush_cylinder
+    from tests.golden.branched_cases import BRANCHED
+    autotune_forget()
+    plain = brush_cylinder(0.5, n_r=43, n_z=101, N=60)
+    try:
+        for t in (plain + "mol : brush : save_memory : true\n", BRANCHED["branch2d_lipid"]["text"]):
+            s = ScfSystem(t)
+            rep = s.autotune(evals=2)
+            assert [c["mode"] for c in rep["candidates"]] == ["grid"] and rep["chosen"] == 0
+            assert s.layout()["mode"] == "grid"
+            s.close()
+        s = ScfSystem(plain)
+        assert s.layout()["mode"] == "fused"
+        autotune_batch([s], evals=1)
+        s.close()
+    finally:
+        autotune_forget()

@@ -103,31 +103,56 @@ def hbm_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     return gf + 8 * M * rows + 8 * diis
 
 
-def recomputed_rows(N, ckpt):
-    """Rows the grid path's backward pass recomputes per evaluation with
-    checkpoint interval K: every row between two checkpoints except those of
-    the last segment, which the forward pass left in the buffer."""
-    if ckpt <= 1:
-        return 0
-    last = (N - 1) // ckpt * ckpt
-    return (N - -(-N // ckpt)) - (N - 1 - last)
+def grid_chain_bytes(N, ckpt, w):
+    """Bytes per site that the launches of a chain of N > 1 segments of one
+    type move on the grid path, up to four propagation steps each (the tiles'
+    halos come from the cache).  A row takes w bytes, segment weights and
+    densities always 8.  Forward steps read their input row and the weights
+    and store the rows that are kept: all, or with checkpoint interval K the
+    checkpoints, the last segment, and each launch's last row in the first
+    pass (launches end at checkpoints for K < 4), and the whole segment when
+    its rows are recomputed.  Backward steps read and write a backward row and
+    the densities and read the weights and every row that they compose."""
+    K = max(1, ckpt)
+    most = 4 // K * K if 1 < K < 4 else 4
+
+    def forward(r0, r1, first):
+        total = 0
+        for r in range(r0, r1, most if first else 4):
+            end = min(r + (most if first else 4), r1)
+            kept = [q for q in range(r + 1, end + 1)
+                    if not first or K == 1 or q % K == 0 or q // K == (N - 1) // K or q == end]
+            total += (w if r > 0 else 8 + w) + 8 + w * len(kept)  # (row 0 is the weight, and stored)
+        return total
+
+    held = (N - 1) // K if K > 1 else 0
+    total = forward(0, N - 1, True) + 8 + w  # the last row: the last segment's weight, composed
+    s, launches = N - 2, 0
+    while s >= 0:
+        if launches and K > 1 and s % K != 0 and s // K != held:
+            held = s // K
+            total += forward(held * K, held * K + K - 1, False)
+        launches += 1
+        n = 0
+        while n < 4 and s >= 0 and (K == 1 or s % K == 0 or s // K == held):
+            n, s = n + 1, s - 1
+        total += (w if launches > 1 else 0) + w + 16 + (8 + n * w if n else 0)
+    return total
 
 
 def grid_bytes_per_evaluation(desc, ckpt=1, w=8, kd=10):
     """Bytes one residual evaluation plus one DIIS update move on the grid
-    path, where a launch takes four propagation steps of every tile (the
-    tiles' halos come from the cache): forward the input row and G1 read once
-    per four steps and every row written, the same for the rows recomputed
-    with checkpoints; backward with composition Gb and G1 read, Gb written
-    and rho read and written per four steps and every Gf row read; over the
-    interior sites.  The per-site arrays of the other phases and the DIIS
+    path: the launches of every chain over the interior sites
+    (grid_chain_bytes), the per-site arrays of the other phases and the DIIS
     history as in hbm_bytes_per_evaluation."""
     W = desc["MX"] * max(1, desc["MY"]) * max(1, desc["MZ"])
-    chains = sum(((2 / 4 + 1 + 5 / 4 + 1) * m["chainlength"] +
-                  (2 / 4 + 1) * recomputed_rows(m["chainlength"], ckpt)) * w * W
-                 for m in desc["molecules"] if m["chainlength"] > 1)
+    long = [m for m in desc["molecules"] if m["chainlength"] > 1]
+    chains = sum(grid_chain_bytes(m["chainlength"], ckpt, w) for m in long) * W
+    # (the weights that the chains read and the densities that they write are
+    # counted there)
     rest = hbm_bytes_per_evaluation(desc, ckpt, w, kd) - \
-        sum(end_point_bytes(desc, m, ckpt, w, W) for m in desc["molecules"])
+        sum(end_point_bytes(desc, m, ckpt, w, W) for m in desc["molecules"]) - \
+        8 * desc["M"] * sum(2 * m["blocks"] + m["molmon"] for m in long)
     return chains + rest
 
 

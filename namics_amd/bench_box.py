@@ -106,6 +106,6 @@ def run_box(args, n=96, seed=41):
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None,
                      "kernel": "whole solve (per-kernel durations in profiles/k_box_box96.md)",
                      "bytes_per_solve": nbytes,
-                     "bytes": "every grid-path launch's streams: 3.75 x 8 B per site and contour step, 1.5 x 8 B per "
-                              "recomputed row, per-site arrays once per evaluation, DIIS history per iteration"},
+                     "bytes": "every grid-path launch's streams (rows read, kept and composed, weights and "
+                              "densities), per-site arrays once per evaluation, DIIS history per iteration"},
     }

@@ -50,6 +50,22 @@ def test_hbm_bytes_count_stored_rows_once_each_way():
     assert bench.hbm_bytes_per_evaluation(d, 1, kd=3) - bench.hbm_bytes_per_evaluation(d, 1, kd=2) == 3 * 8 * 25740
 
 
+def test_grid_bytes_count_the_rows_of_every_launch():
+    # 20 segments, a checkpoint every 4: forward five launches (row 0 and 4
+    # rows read, weights five times, 8 rows kept); the three segments before
+    # the last recomputed from a row, the first from the weight (3 rows kept
+    # each, row 0 once more); five backward launches over 20 rows
+    for w in (8, 4):
+        forward = 8 + 4 * w + 5 * 8 + 8 * w
+        recompute = 3 * (w + 8 + 3 * w) + (8 + 8 + w + 3 * w)
+        backward = (8 + 4 * w) + 5 * (w + 8 + 16) + 20 * w
+        assert bench.grid_chain_bytes(20, 4, w) == forward + recompute + backward
+    # every row kept, 13 segments: three launches each way
+    assert bench.grid_chain_bytes(13, 1, 8) == (8 + 2 * 8) + 3 * 8 + 13 * 8 + (8 + 2 * 8) + 3 * (8 + 8 + 16) + 13 * 8
+    # two segments: one launch each way
+    assert bench.grid_chain_bytes(2, 1, 8) == 8 + 8 + 2 * 8 + 8 + (8 + 8 + 16) + 2 * 8
+
+
 def test_compare_with_reference_counts_both_and_free_energy():
     ref = {3: [{"residual": 5e-8, "free_energy": -2.0}, {"residual": 1e-3, "free_energy": 1.0},
                {"residual": 9e-8, "free_energy": 4.0}]}

@@ -197,11 +197,13 @@ double fraction(const MoleculeSpec &m, int seg) {
 // lattice.  Time in strips over time in registers, one residual evaluation,
 // N = 200, MX 32 .. 128 (a row each where it fits):
 //   strips of 8   MY 32 0.76-0.83, 48 0.88-0.94, 60 0.94-1.05, 64 1.04-1.14,
-//                 65-76 0.95-1.07, 80 0.99-1.07, 84 1.01-1.11, 96 1.03-1.14,
-//                 128 1.28-1.33, 129 1.03, 192 1.14, 256 1.21
+//                 65-80 0.95-1.07 up to 4200 sites and 1.02-1.06 above, 84
+//                 1.01-1.11, 96 1.03-1.14, 128 1.28-1.33, 129 1.03, 192 1.14,
+//                 256 1.21
 //   strips of 4   MY 32 0.60-0.70, 64 0.78-0.89, 96 0.96, 112 0.99
-// 256 systems at once are up to a tenth faster in registers at 65 to 80 layers.
-bool registers_faster(int sx, int MY) { return sx == 8 && (MY == 64 || MY >= 84); }
+bool registers_faster(int sx, int MX, int MY) {
+  return sx == 8 && (MY == 64 || MY >= 84 || (MY > 64 && MX * MY > 4200));
+}
 
 // Launch layout of the fused path: threads per system, whether the
 // propagator rows live in LDS, and on 2-gradient lattices the register-strip
@@ -271,7 +273,7 @@ void plan_layout(scf_system *S, int want_sx, int registers) {
   if (yp > 0) {
     const int nw = (l.MX + kWave2Sites / yp - 1) / (kWave2Sites / yp);
     const size_t edges = (size_t)2 * nw * 128 * yp * D, own = (size_t)1024 * kWave2Sites * D;
-    if (nw <= 16 && edges <= lds_limit() && (registers == 1 || h.strip_sx == 0 || registers_faster(h.strip_sx, l.MY))) {
+    if (nw <= 16 && edges <= lds_limit() && (registers == 1 || h.strip_sx == 0 || registers_faster(h.strip_sx, l.MX, l.MY))) {
       h.wave2 = yp;
       h.wave2_own = edges + own <= lds_limit() ? 1 : 0;
       h.threads = std::max(h.threads, 64 * nw);
@@ -504,7 +506,6 @@ int build(scf_system *S, const Placement *pl) {
   size_t o_x = a.take(nvar * D);
   size_t o_g = a.take(nvar * D);
   size_t o_G1 = a.take((size_t)nseg * M * D);
-  // FP32 segment weights of the grid path's mixed-precision chains (3 gradients)
   // end-point rows; the 1-gradient tiles pad theirs to whole waves, which on
   // a small lattice is more than the rows themselves
   size_t gf_doubles = (size_t)maxNR * M;

@@ -287,7 +287,7 @@ def run_brush(args):
         probe.close()
     slots = [[ScfSystem(brush_cylinder(c)) for c in CHIS] for _ in range(nslots)]
     # end-point storage: tuned with all slots in flight (every row, or every
-    # other row with the odd rows recomputed on chip), unless given
+    # second or third with the others recomputed on chip), unless given
     ck = args.checkpoint
     if ck == 0 and not args.no_tune:
         tune_batch = autotune_batch([row[0] for row in slots])

@@ -194,13 +194,13 @@ int scf_system_autotune(scf_system *sys, int evals, scf_tune_report *report);
  * workgroup per system, as scf_solve_resident and the job queue run them).
  * Times `evals` residual evaluations of all n systems in one launch for each
  * end-point storage that applies -- every row (interval 1) and, when every
- * system is on the 2-gradient strip path, every other row with the odd rows
- * recomputed on chip (interval 2, scf_system_set_checkpoint), and, where
- * those rows together exceed the last-level cache, every third (interval 3)
- * -- and applies the fastest to all n.  Alone, a system's propagation is bound by its own
- * LDS traffic and recomputing rows costs time; with one system per CU the
- * stored rows saturate HBM and halving them pays.  Results are bit-identical
- * either way.  No counterpart in the reference. */
+ * system has a 2-gradient strip layout, every other row with the odd rows
+ * recomputed on chip (interval 2, scf_system_set_checkpoint), and, where all
+ * keep their lattice in registers and those rows together exceed the
+ * last-level cache, every third (interval 3) -- and applies the fastest to
+ * all n.  Alone, a system's propagation is bound by its serial steps on one
+ * CU and recomputing rows costs time; with one system per CU the stored rows
+ * saturate HBM and keeping fewer pays.  Results are bit-identical either way.  No counterpart in the reference. */
 typedef struct {
   int candidates;
   int chosen;
@@ -210,8 +210,13 @@ typedef struct {
 int scf_autotune_batch(scf_system *const *systems, int n, int evals, scf_batch_tune_report *report);
 /* Forget the layouts remembered per lattice shape (tests, benchmarks). */
 void scf_autotune_forget(void);
-/* The system's current launch layout: execution mode, strip width (0 when
- * not on the strip path) and threads per system. */
+/* The system's current launch layout: the execution mode its settings and
+ * options give, the strip width (0 when no strip fits; next to the lattice in
+ * registers, the width of the FP32 chains) and threads per system.  In
+ * SCF_MODE_AUTO a call can still take another path than this mode: a branched
+ * 1-gradient system, reported as the grid path, runs in one workgroup where
+ * its rows fit LDS and no end points are checkpointed, and a few 2-gradient
+ * systems whose rows do not fit LDS, reported as fused, run on the grid path. */
 int scf_system_layout(const scf_system *sys, int *mode, int *strip_sx, int *threads);
 
 /* ---- output and format layer (the reference's files) ----

@@ -30,8 +30,8 @@ namespace nscf {
 // Measured on one MI355X, chains per evaluation: 64 x 128, N = 200, one
 // system 0.68 -> 0.44 ms (1.1 us per step, half of it the 72 vector
 // instructions of 4 waves per SIMD, the rest the LDS exchange and its
-// barrier); 256 systems 1.04 (interval 2) -> 0.75 ms (interval 3); 43 x 101,
-// N = 120, which the strips cannot divide, 1.32 -> 0.25 ms.
+// barrier); 256 systems 1.04 (interval 2) -> 0.65 ms (interval 3); 43 x 101,
+// N = 120, which the strips cannot divide, 1.34 -> 0.26 ms.
 template <int YP, bool kFull>
 struct Wave2 {
   static constexpr int SX = kWave2Sites / YP;

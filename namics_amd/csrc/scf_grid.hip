@@ -1,7 +1,8 @@
 // Multi-workgroup SCF path for lattices too large for one workgroup
 // (3-gradient boxes such as 96^3): each phase of a residual evaluation is a
-// grid-stride kernel, each propagation step one launch over all sites, and
-// the DIIS loop is driven from the host with one small readback (status and
+// grid-stride kernel; the chains of the 6-point 3-gradient stencil and of
+// 2-gradient lattices run as tiles, several propagation steps per launch
+// (scf_box3d.h, scf_tile2d.h), other chains one launch per step; the DIIS loop is driven from the host with one small readback (status and
 // residual) per iteration.  The per-site arithmetic is shared with the fused
 // kernel (scf_device.h).  Reductions are deterministic: per-workgroup
 // partial sums in HBM, summed in workgroup order by one thread.
